@@ -1500,7 +1500,6 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     };
 
     const uint32_t cus = c->cus;
-    const dim3 trace_grid(cus * c->tune.trace_blocks_per_cu);
     uint64_t iterations = 0;
     KernelTimer kt{c, timing, s};
     uint64_t items_done_before = 0;
@@ -1551,7 +1550,17 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         }
         HIP_TRY(c, hipStreamSynchronize(s));
         if (multi) hipLaunchKernelGGL(k_clock_stamp, dim3(1), dim3(64), 0, s, d_ticks + djobs.size());
-        const dim3 g_shade(std::min<uint32_t>((P.nslots + kBlock - 1) / kBlock, cus * c->tune.shade_blocks_per_cu));
+        /* Slots that can still hold a path: all of them at first, then what the last counter readback found (a slot
+         * without a work item never gets one again, so the count only falls).  Launches are sized to it: a lane per
+         * ray, up to the tuned block counts.  A trace block without a ray still takes queue counters from the others
+         * (same-address atomics) and scans all shards before it ends. */
+        uint32_t live = P.nslots;
+        dim3 trace_grid, g_shade;
+        auto size_grids = [&]() {
+            trace_grid = dim3(std::min<uint32_t>((live + kTraceBlock - 1) / kTraceBlock, cus * c->tune.trace_blocks_per_cu));
+            g_shade = dim3(std::min<uint32_t>((live + kBlock - 1) / kBlock, cus * c->tune.shade_blocks_per_cu));
+        };
+        size_grids();
 
         /* one wavefront iteration: extend, shade (+ cache queries), shadow, secondary walks, finish / refill */
         auto iteration = [&](auto mt, uint32_t cur) -> vvpt_status {
@@ -1643,6 +1652,10 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                 const uint64_t done = items_done_before + (started > active ? started - active : 0);
                 c->progress.store((float)((double)done / (double)total_items));
                 if (active == 0u) break;
+                if (!gx) { /* a captured graph keeps its grids */
+                    live = (uint32_t)std::min<uint64_t>(active, P.nslots);
+                    size_grids();
+                }
                 if (window_iters >= max_iters) {
                     v = set_err(c, VVPT_TIMEOUT, "render did not finish within " + std::to_string(max_iters) +
                                                      " wavefront iterations");
