@@ -9,17 +9,17 @@
  * state carried across samples (rng_def.glsl:32-36, raygen.rgen.glsl:37,55), and
  * every iteration of the host loop advances all active slots by one bounce:
  *
+ *   k_secondary  shadow segments and emitter-lookup walks of the previous bounce that need the general walk (any-hit
+ *                logic applied closest-first)
+ *   k_shadow     single-segment shadow rays of the previous bounce
  *   k_extend     closest-hit query of each slot's ray; when the previous bounce
  *                asked for a BSDF-direction emitter lookup (next_event_estimation.glsl)
  *                the same walk also answers it (MODE_CLOSEST2)
- *   k_shade      one bounce of the closest-hit / miss shaders; light sampling
- *                and emitter lookups that need their own walk become records
- *                in a secondary queue
- *   k_secondary  shadow segments and emitter-lookup walks (any-hit logic
- *                applied closest-first)
- *   k_finish     adds secondary results in a fixed order, ends samples, writes
- *                finished work items, regenerates camera rays and compacts the
- *                next queue (wave ballot + prefix count, one atomic per wave)
+ *   k_shade      adds the previous bounce's secondary results in a fixed order, then one bounce of the closest-hit /
+ *                miss shaders; light sampling and emitter lookups that need their own walk become records in a
+ *                shadow or secondary queue; samples that end are accumulated, finished work items written and
+ *                replaced, camera rays regenerated, and the next queue compacted (wave ballot + prefix count, one
+ *                atomic per wave)
  *
  * Results of a work item depend only on (pixel, batch), so the image is the
  * same whatever the slot scheduling; k_resolve sums the per-batch partials in
@@ -44,7 +44,7 @@ constexpr int kBlock = 256;
 
 enum : uint32_t {
     F_NEE = 1u,        /* the slot's ray also carries the previous bounce's emitter lookup */
-    F_DONE = 2u,       /* the sample ended in k_shade */
+    F_DONE = 2u,       /* the sample is over and waits for the results named by the other bits (parked) */
     F_SEC0 = 4u,       /* secondary record 0 (shadow ray) pending */
     F_SEC1 = 8u,       /* secondary record 1 (emitter lookup of the previous bounce) pending */
     F_SEC2 = 16u,      /* secondary record 2 (emitter lookup of the last bounce) pending */
@@ -55,7 +55,10 @@ enum : uint32_t {
                              estimate there exceeds its tolerance, so it continues */
 };
 
-/* stats[] slots (64-bit) */
+/* Extension-queue entries are slots; an entry with this bit set has no ray to trace: its sample is over but waits for
+ * results still being computed (shadow records, a cache query), which the next k_shade adds before it ends it. */
+constexpr uint32_t kParked = 0x80000000u;
+
 /* stats[] slots (64-bit); each wave adds into the copy of its shard (kStatStride apart) */
 enum : uint32_t {
     S_PATH = 0, S_SHADOW = 1, S_NEE = 2, S_NODES_EXT = 3, S_TRIS_EXT = 4, S_NODES_SEC = 5, S_TRIS_SEC = 6,
@@ -132,12 +135,13 @@ struct PathState {
 struct RenderParams {
     uint32_t items_total; /* work items of this launch window (all jobs) */
     uint32_t aovs;
+    uint32_t media;    /* a path can be inside a medium (Features::vol): the slots' volumes are kept */
     uint32_t extended; /* extended mode: scrambled Sobol samples, environment importance sampling */
     uint32_t nslots;
     float total_samples;
     SQueue ext[2]; /* slots with a ray to extend (double-buffered across iterations) */
     SQueue sec;    /* secondary records needing a general walk (3 per slot) */
-    SQueue shd;    /* single-segment shadow rays (scenes without volume-changing surfaces) */
+    SQueue shd[2]; /* single-segment shadow rays (scenes without volume-changing surfaces), double-buffered like ext */
     uint32_t *items; /* kShards padded work-item counters */
     uint32_t items_per_shard;
     uint32_t item_chunk; /* 0: contiguous item shards; else chunks of this many items dealt round-robin */
@@ -229,7 +233,7 @@ __device__ __forceinline__ void nrc_emit_training(const RenderParams &P, uint32_
 
 /* Radiance-cache state of a starting sample: a small hashed fraction of samples trains the cache (their paths
  * are traced to the end and every surface vertex is recorded), the others may end in a cache query. */
-__device__ __forceinline__ void nrc_sample_start(const RenderParams &P, const JobView &J, PathState &st, uint32_t slot,
+__device__ __forceinline__ void nrc_sample_start(const RenderParams &P, const JobView &J, const PathState &st, uint32_t slot,
                                                  uint32_t item, uint32_t sample) {
     uint32_t t = kInvalid;
     const uint32_t bl = item / J.npix, pix = item - bl * J.npix;
@@ -242,12 +246,23 @@ __device__ __forceinline__ void nrc_sample_start(const RenderParams &P, const Jo
     st.spread[slot] = make_float2(0.0f, 0.0f);
 }
 
+/* What a render can meet, fixed when k_shade is compiled: a kernel that carries every estimator's code for every
+ * scene is 170 KB of instructions (more than the instruction cache of two CUs) and keeps its kernel arguments in
+ * spilled registers. */
+template <bool EXT_, bool NRC_, bool TEX_, bool VOL_>
+struct Features {
+    static constexpr bool ext = EXT_; /* the extended estimator (scrambled Sobol samples, environment sampling) */
+    static constexpr bool nrc = NRC_; /* the radiance cache (with ext) */
+    static constexpr bool tex = TEX_; /* some surface has a texture of its own besides the alpha cut-out */
+    static constexpr bool vol = VOL_; /* a path can be inside a medium: the camera is, or a surface bounds one */
+};
+
 /* Generator of sample `sample` of the job's work item `item` (parity: the stored xorshift state). */
-__device__ __forceinline__ Rng rng_of(const RenderParams &P, const JobView &J, uint32_t state, uint32_t item,
-                                      uint32_t sample) {
+template <class Fx>
+__device__ __forceinline__ Rng rng_of(const JobView &J, uint32_t state, uint32_t item, uint32_t sample) {
     Rng r;
     r.s = state;
-    r.ld = P.extended != 0u;
+    r.ld = Fx::ext;
     r.n = 0u;
     r.key = 0u;
     if (r.ld) {
@@ -475,6 +490,12 @@ __device__ __forceinline__ void hit_geometry(const DInstance &I, const Tri3 &T, 
     g.flipped = fixFrame(g.frame.normal, g.frame.tangent, g.frame.bitangent, rayDir);
 }
 
+/* Emission with the texture product left out where every emissive slot holds the default white texel (x * 1 = x). */
+template <class Fx>
+__device__ __forceinline__ f3 mat_emissive_fx(const DScene &S, const DMaterial &m, float tu, float tv) {
+    if (!Fx::tex) return m.emissive[3] * mk(m.emissive[0], m.emissive[1], m.emissive[2]);
+    return m.emissive[3] * mk(m.emissive[0], m.emissive[1], m.emissive[2]) * tex_rgb(S, m.tex2[0], tu, tv);
+}
 __device__ __forceinline__ f3 mat_emissive(const DScene &S, const DMaterial &m, float tu, float tv) {
     return m.emissive[3] * mk(m.emissive[0], m.emissive[1], m.emissive[2]) * tex_rgb(S, m.tex2[0], tu, tv);
 }
@@ -576,6 +597,7 @@ struct CandInfo {
     bool vol_change;
     f3 emissive;
 };
+template <class Fx = Features<true, true, true, true>>
 __device__ __forceinline__ CandInfo cand_info(const DScene &S, const TraceHit &h, bool need_emissive) {
     const DInstance &I = S.insts[h.inst];
     const DMaterial &m = S.inst_mats[h.inst];
@@ -592,7 +614,7 @@ __device__ __forceinline__ CandInfo cand_info(const DScene &S, const TraceHit &h
         hit_uv(Tr, mk(1.0f - h.u - h.v, h.u, h.v), u, v);
         const float tu = u * m.tiling[0], tv = v * m.tiling[1];
         if (c.transparent) c.alpha = mat_alpha(S, m, tu, tv);
-        if (need_emissive && (m.flags & 1u)) c.emissive = mat_emissive(S, m, tu, tv);
+        if (need_emissive && (m.flags & 1u)) c.emissive = mat_emissive_fx<Fx>(S, m, tu, tv);
     }
     return c;
 }
@@ -616,8 +638,8 @@ __device__ __forceinline__ void cross_volume_surface(const DScene &S, const Trac
 }
 
 /* ------------------------------------------------------------ k_init -- */
-template <bool MULTI>
-__device__ __forceinline__ void start_item(const DScene &S, const RenderParams &P, PathState &st, uint32_t slot,
+template <bool MULTI, class Fx>
+__device__ __forceinline__ void start_item(const DScene &S, const RenderParams &P, const PathState &st, uint32_t slot,
                                                uint32_t gitem) {
     uint32_t item = gitem;
     if (MULTI) {
@@ -629,13 +651,13 @@ __device__ __forceinline__ void start_item(const DScene &S, const RenderParams &
     const uint32_t bl = item / J.npix, pix = item - bl * J.npix;
     const uint32_t px = pix % J.W, py = pix / J.W;
     /* parity: the batch's stream starts here (raygen.rgen.glsl:37); extended: dimension 0 of sample 0 */
-    Rng rng = rng_of(P, J, P.extended ? 0u : initRNG(px, py, J.W, J.batch_begin + bl, J.seed), item, 0u);
+    Rng rng = rng_of<Fx>(J, Fx::ext ? 0u : initRNG(px, py, J.W, J.batch_begin + bl, J.seed), item, 0u);
     f3 o, d;
     camera_ray(J, px, py, rng, o, d);
     st.rng[slot] = rng.s;
-    if (P.nrc) nrc_sample_start(P, J, st, slot, item, 0u);
+    if (Fx::nrc && P.nrc) nrc_sample_start(P, J, st, slot, item, 0u);
     st.ctr[slot] = ctr_make(0, 0, 0);
-    st.vol[slot] = J.cam_volume >= 0 ? (uint32_t)J.cam_volume : kInvalid;
+    if (Fx::vol) st.vol[slot] = J.cam_volume >= 0 ? (uint32_t)J.cam_volume : kInvalid;
     st.orig[slot] = st4(o, 0.0f);
     st.dir[slot] = st4(d, 0.0f);
     st.beta[slot] = make_float4(1.f, 1.f, 1.f, -1.f); /* w: last scattering pdf, -1 none */
@@ -644,12 +666,12 @@ __device__ __forceinline__ void start_item(const DScene &S, const RenderParams &
     if (P.aovs) {
         st.accA[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
         st.accN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
+        st.payA[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
+        st.payN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    st.payA[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
-    st.payN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-template <bool MULTI>
+template <bool MULTI, class Fx>
 __global__ __launch_bounds__(kBlock) void k_init(DScene S, RenderParams P, PathState st) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t i0 = i & ~63u;
@@ -661,7 +683,7 @@ __global__ __launch_bounds__(kBlock) void k_init(DScene S, RenderParams P, PathS
         st.item[i] = item;
         st.flags[i] = 0u;
         if (item != kInvalid) {
-            start_item<MULTI>(S, P, st, i, item);
+            start_item<MULTI, Fx>(S, P, st, i, item);
             active = true;
         }
     }
@@ -673,7 +695,11 @@ template <int STACK, bool COUNT, bool MULTI>
 __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(DScene S, RenderParams P, PathState st, uint32_t cur) {
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
     uint2 *my = stack + threadIdx.x;
+    /* the queues that this iteration's k_shade fills; their last consumers ran before this kernel */
     sq_reset(P.ext[cur ^ 1u]);
+    sq_reset(P.shd[cur ^ 1u]);
+    sq_reset(P.sec);
+    if (P.nrc_use) sq_reset(P.nrcq);
     const SQueue &Q = P.ext[cur];
     uint32_t nrays = 0;
     TraceCount cnt = {0, 0};
@@ -682,7 +708,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(DSc
     uint32_t shard = wave_global_id() % kShards, slot = 0;
     for (;;) {
         uint32_t v = 0;
-        if (sq_refill(Q, !active, shard, done, v) && !active) {
+        if (sq_refill(Q, !active, shard, done, v) && !active && !(v & kParked)) {
             slot = v;
             const f3 O = ld3(st.orig[slot]), D = ld3(st.dir[slot]);
             const uint32_t fl = st.flags[slot];
@@ -729,6 +755,7 @@ struct LightSample {
     float pdf, tmax;
     bool delta;
 };
+template <class Fx>
 __device__ __forceinline__ LightSample sample_light(const DScene &S, const JobView &J, Rng &rng, f3 P, bool env_last) {
     LightSample ls;
     ls.delta = true;
@@ -740,7 +767,7 @@ __device__ __forceinline__ LightSample sample_light(const DScene &S, const JobVi
     if (total == 0u) return ls;
     const float pdf = 1.0f / (float)total;
     const uint32_t li = min((uint32_t)(rnd(rng) * (float)total), total - 1u);
-    if (li >= J.num_lights) {
+    if (Fx::ext && li >= J.num_lights) {
         /* extended mode: an environment sample, shadowed like a directional light */
         const float u0 = rnd(rng), u1 = rnd(rng), u2 = rnd(rng), u3 = rnd(rng);
         f3 dir;
@@ -800,7 +827,7 @@ __device__ __forceinline__ LightSample sample_light(const DScene &S, const JobVi
         ls.dir = dv / ls.tmax;
         const float dp = dot(-ls.dir, sn);
         if (dp > 0.0f) {
-            ls.radiance = mat_emissive(S, m, su * m.tiling[0], sv * m.tiling[1]);
+            ls.radiance = mat_emissive_fx<Fx>(S, m, su * m.tiling[0], sv * m.tiling[1]);
             ls.pdf = pdf * trianglePdf * sampledPointPdf * distanceSquared(P, sp) / dp;
         } else {
             ls.radiance = {0, 0, 0};
@@ -814,13 +841,13 @@ __device__ __forceinline__ LightSample sample_light(const DScene &S, const JobVi
 /* Storage index of secondary record r = 3 slot + k. */
 __device__ __forceinline__ uint32_t sec_ix(const PathState &st, uint32_t r) { return (r % 3u) * st.nsec + r / 3u; }
 
-__device__ __forceinline__ void emit_sec(const RenderParams &P, PathState &st, uint32_t slot, uint32_t k, f3 o,
+__device__ __forceinline__ void emit_sec(const RenderParams &P, const PathState &st, uint32_t slot, uint32_t k, f3 o,
                                          float w_o, f3 d, float w_d, f3 c, uint32_t vol) {
     const uint32_t r = k * st.nsec + slot;
     st.sec_o[r] = st4(o, w_o);
     st.sec_d[r] = st4(d, w_d);
     st.sec_c[r] = st4(c, 0.0f);
-    st.sec_v[r] = vol;
+    if (P.media) st.sec_v[r] = vol;
 }
 
 /* process_volume_hit.glsl:1-45 (sampling part).  Returns sampledMedium, updates beta. */
@@ -849,25 +876,27 @@ __device__ __forceinline__ bool volume_sample(const DScene &S, uint32_t volIdx, 
     return sampled;
 }
 
-/* One bounce of slot `slot`; returns the mask of secondary records it wrote. */
-__device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J, const RenderParams &P, PathState &st,
-                                              uint32_t slot) {
+/* One bounce of slot `slot`, whose flags word is flags_in and whose radiance so far is L.  Returns the mask of
+ * secondary records it wrote (and F_NRCQ, F_NRC_FALLBACK); `over` is set when the sample has ended.  A sample that
+ * ends with nothing pending leaves no state behind but its radiance in L and its generator state in rng_out. */
+template <class Fx>
+__device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J, const RenderParams &P, const PathState &st,
+                                              uint32_t slot, uint32_t flags_in, uint32_t ctr, f3 &L, uint32_t &rng_out,
+                                              bool &over) {
     {
-        const uint32_t flags_in = st.flags[slot];
         uint32_t flags = flags_in & F_NEE;
-        const uint32_t ctr = st.ctr[slot];
-        Rng rng = rng_of(P, J, st.rng[slot], P.extended ? st.item[slot] - J.item_begin : 0u, ctr_sample(ctr));
+        Rng rng = rng_of<Fx>(J, st.rng[slot], Fx::ext ? st.item[slot] - J.item_begin : 0u, ctr_sample(ctr));
         const uint32_t d = ctr_depth(ctr);
         uint32_t sdepth = ctr_sdepth(ctr);
-        uint32_t vol = st.vol[slot];
-        bool inside = vol != kInvalid;
+        uint32_t vol = kInvalid;
+        if (Fx::vol) vol = st.vol[slot];
+        bool inside = Fx::vol && vol != kInvalid;
         const float4 beta4 = st.beta[slot];
         f3 beta = ld3(beta4);
         /* extended mode: pdf of the direction sampled at the last scattering vertex (-1: a camera ray), the BSDF
          * side of the MIS pair for environment light found by this ray */
         float misp = beta4.w;
         const bool env_last = d + 1u >= J.depth; /* no environment sample where the BSDF side cannot follow */
-        f3 L = ld3(st.L[slot]);
         const f3 O = ld3(st.orig[slot]);
         const f3 D = ld3(st.dir[slot]);
         uint32_t secmask = 0;
@@ -880,7 +909,7 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
             /* hA is the first candidate that is not passed (INST_NEE_PASS instances are transparent,
              * non-emissive and keep the volume: rayNEE.rahit.glsl:43-70 only scales their throughput) */
             if (hA.prim != kInvalid && hA.t <= J.zfar) {
-                const CandInfo c = cand_info(S, hA, true);
+                const CandInfo c = cand_info<Fx>(S, hA, true);
                 if (isBlackEps(c.emissive, 0.05f)) {
                     if (c.transparent) {
                         /* a transparent surface that changes volume (or whose emission texture is black
@@ -909,8 +938,8 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
         }
         if (flags_in & F_TERMINAL) {
             /* the walk only answered the last bounce's emitter lookup: the sample is over */
-            st.L[slot] = st4(L, 0.f);
-            st.flags[slot] = F_DONE | secmask;
+            rng_out = rng.s;
+            over = true;
             return secmask;
         }
 
@@ -923,16 +952,16 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
         f3 neeBeta = {0, 0, 0};
         bool sampledMedium = false;
         float vhd = 0.0f, g = 0.0f;
-        if (inside) {
+        if (Fx::vol && inside) {
             const float vtend = h.prim != kInvalid ? h.t : fminf((float)(uint32_t)J.zfar, 10000.0f);
             sampledMedium = volume_sample(S, vol, rng, beta, 0.001f, vtend, vhd, g);
         }
-        if (sampledMedium) {
+        if (Fx::vol && sampledMedium) {
             /* process_volume_hit.glsl:42-79: scattering event */
             const f3 wrd = normalize(D);
             const f3 wo = -wrd;
             const f3 sp = O + (0.001f + vhd) * wrd;
-            const LightSample ls = sample_light(S, J, rng, sp, env_last);
+            const LightSample ls = sample_light<Fx>(S, J, rng, sp, env_last);
             if (!isBlack(ls.radiance)) {
                 const float p = HenyeyGreenstein(dot(wo, ls.dir), g);
                 if (p != 0.0f) {
@@ -960,27 +989,23 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
             stop = true;
             do_rr = false;
             const f3 bg = mk(S.bg[0], S.bg[1], S.bg[2]);
-            if (S.env_type == 0u) {
-                if (sdepth == 0u) {
-                    st.payA[slot] = st4(bg, 0.f);
-                    st.payN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-                L = L + bg * beta;
-            } else if (S.env_type == 1u) {
-                const f3 c = S.env_intensity * env_lookup(S, D);
-                if (sdepth == 0u) {
+            /* the environment's radiance along the ray: the background colour (type 0, and camera rays of type 2), the
+             * map (scaled by the intensity for type 1) */
+            f3 c = bg;
+            const bool map = S.env_type == 1u || (S.env_type == 2u && sdepth != 0u);
+            if (map) {
+                c = env_lookup(S, D);
+                if (S.env_type == 1u) c = S.env_intensity * c;
+            }
+            if (S.env_type <= 2u) {
+                if (P.aovs && sdepth == 0u) {
                     st.payA[slot] = st4(c, 0.f);
                     st.payN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
-                L = L + env_mis(S, J, misp, D) * c * beta;
-            } else if (S.env_type == 2u) {
-                if (sdepth == 0u) {
-                    st.payA[slot] = st4(bg, 0.f);
-                    st.payN[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    L = L + bg * beta;
-                } else {
-                    L = L + env_mis(S, J, misp, D) * env_lookup(S, D) * beta;
-                }
+                if (Fx::ext && map)
+                    L = L + env_mis(S, J, misp, D) * c * beta;
+                else
+                    L = L + c * beta;
             }
         } else {
             /* rayPrimary{Lambert,PBRStandard}.rchit.glsl:60-172 */
@@ -997,7 +1022,7 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
                 const float alpha = mat_alpha(S, m, tu, tv);
                 const float ra = rnd(rng);
                 if (alpha < EPSILON || ra > alpha) {
-                    if (I.idg != I.idb) {
+                    if (Fx::vol && I.idg != I.idb) {
                         inside = false;
                         const float nv = gg.flipped ? I.idg : I.idb;
                         if (nv != -1.0f) {
@@ -1014,16 +1039,20 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
             }
             if (!passed) {
                 Frame fr = gg.frame;
-                applyNormalToFrame(fr, processNormalFromNormalMap(tex_rgb(S, m.tex2[1], tu, tv)));
-                const f3 albedo = mk(m.albedo[0], m.albedo[1], m.albedo[2]) * tex_rgb(S, m.tex1[0], tu, tv);
+                /* without textures every slot holds its default texel: white (x * 1 = x) or the flat normal */
+                applyNormalToFrame(fr, processNormalFromNormalMap(
+                                           Fx::tex ? tex_rgb(S, m.tex2[1], tu, tv)
+                                                   : mk(S.flat_normal[0], S.flat_normal[1], S.flat_normal[2])));
+                f3 albedo = mk(m.albedo[0], m.albedo[1], m.albedo[2]);
+                if (Fx::tex) albedo = albedo * tex_rgb(S, m.tex1[0], tu, tv);
                 PBRStd pbr;
                 if (isPBR) {
                     pbr.albedo = albedo;
-                    pbr.metallic = m.mra[0] * tex_sample(S, m.tex1[1], tu, tv).x;
-                    pbr.roughness = fmaxf(m.mra[1] * tex_sample(S, m.tex1[2], tu, tv).x, 0.035f);
+                    pbr.metallic = Fx::tex ? m.mra[0] * tex_sample(S, m.tex1[1], tu, tv).x : m.mra[0];
+                    pbr.roughness = fmaxf(Fx::tex ? m.mra[1] * tex_sample(S, m.tex1[2], tu, tv).x : m.mra[1], 0.035f);
                 }
-                const f3 emissive = (m.flags & 1u) ? mat_emissive(S, m, tu, tv) : mk(0, 0, 0);
-                if (sdepth == 0u) {
+                const f3 emissive = (m.flags & 1u) ? mat_emissive_fx<Fx>(S, m, tu, tv) : mk(0, 0, 0);
+                if (sdepth == 0u && P.aovs) {
                     st.payA[slot] = st4(albedo, 0.f);
                     st.payN[slot] = st4(fr.normal * 0.5f + mk(0.5f, 0.5f, 0.5f), 0.f);
                 }
@@ -1034,7 +1063,7 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
                 } else {
                     sdepth += 1u;
                     bool cached = false;
-                    if (P.nrc) {
+                    if (Fx::nrc && P.nrc) {
                         /* path spread (Müller et al. 2021): footprint a0 = d^2 / (4 pi cos) at the primary vertex,
                          * then sum of sqrt(d^2 / (p cos)) over the vertices after it */
                         const float cosn = fmaxf(fabsf(dot(fr.normal, D)), 1e-4f);
@@ -1073,9 +1102,16 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
                             secmask |= F_NRCQ;
                         }
                     }
-                    const f3 wo = worldToLocal(fr, -D);
+                    f3 wo = worldToLocal(fr, -D);
+                    {
+                        /* the cosine with its rounding fixed (the last product is rounded before it is added), so that
+                         * every Features variant makes the same image whatever else the compiler can share it with */
+#pragma clang fp contract(off)
+                        const float xy = __fmaf_rn(D.y, fr.normal.y, D.x * fr.normal.x);
+                        wo.y = -(xy + D.z * fr.normal.z);
+                    }
                     const LightSample ls = cached ? LightSample{{0, 0, 0}, {0, 0, 0}, 1.0f, 0.0f, true}
-                                                  : sample_light(S, J, rng, gg.wp, env_last);
+                                                  : sample_light<Fx>(S, J, rng, gg.wp, env_last);
                     if (!isBlack(ls.radiance)) {
                         const f3 wi = worldToLocal(fr, ls.dir);
                         f3 F;
@@ -1159,51 +1195,200 @@ __device__ __forceinline__ uint32_t shade_one(const DScene &S, const JobView &J,
             st.nee[slot] = st4(neeBeta, neePdf);
             flags |= F_NEE | F_TERMINAL;
         } else {
-            flags |= F_DONE;
+            over = true;
+            rng_out = rng.s;
+            if (secmask & F_NRCQ) st.beta[slot] = st4(beta, misp); /* the query's weight */
+            return secmask;
         }
         st.beta[slot] = st4(beta, misp);
         st.L[slot] = st4(L, 0.f);
         st.rng[slot] = rng.s;
-        st.vol[slot] = inside ? vol : kInvalid;
+        if (Fx::vol) st.vol[slot] = inside ? vol : kInvalid;
         st.flags[slot] = flags | (secmask & ~F_NRC_FALLBACK);
         return secmask;
     }
 }
 
-template <bool MULTI>
-/* k_shade needs 179 VGPRs unconstrained (2 waves per SIMD); capped at 168 it runs 3 waves without spilling, which
- * hides more of its dependent gathers (55 -> 50 ms per 1080p frame at 64 spp). */
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(DScene S, RenderParams P, PathState st, uint32_t cur) {
+/* Completion bookkeeping of a batched render: the lanes of a wave that ended a work item subtract their count from
+ * their job's remaining items with one atomic per job present in the wave (same-address atomics serialize in L2,
+ * and every item of a large job would otherwise hit the one counter); the lane that takes a counter to zero stamps
+ * the job's completion time.  Called in wave-uniform control flow; `job` is kInvalid for lanes that ended nothing. */
+__device__ __forceinline__ void job_items_done(const DScene &S, uint32_t job) {
+    unsigned long long m = __ballot(job != kInvalid);
+    const uint32_t lane = __lane_id();
+    while (m != 0ull) {
+        const int leader = __ffsll((long long)m) - 1;
+        const uint32_t lj = __shfl(job, leader);
+        const unsigned long long same = __ballot(job == lj);
+        if ((int)lane == leader) {
+            const uint32_t n = (uint32_t)__popcll(same);
+            const JobView &J = S.jobs[lj];
+            if (atomicSub(J.remaining, n) == n) *J.done_ticks = wall_clock64();
+        }
+        m &= ~same;
+    }
+}
+
+/* Arguments of k_shade, read where they are used: a by-value kernel argument is loaded whole at the kernel's entry and
+ * held in scalar registers to its end, and these 900 bytes spilled 229 of them (2,600 v_readlane in the code).  The
+ * empty asm keeps the loads behind this point; they are scalar loads from the constant kernel-argument segment. */
+struct ShadeArgs {
+    DScene S;
+    RenderParams P;
+    PathState st;
+    uint32_t cur;
+};
+template <class T>
+__device__ __forceinline__ const T &kernargs() {
+    const __attribute__((address_space(4))) char *p =
+        (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const T *)(const char *)p;
+}
+
+/* Second half of k_shade for one wave's slots (shard sh, every lane calls it): ends the samples that are over
+ * (raygen.rgen.glsl:126-128), refills ended work items and appends the slots that go on to the next queue. */
+template <bool MULTI, class Fx>
+__device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool valid, bool over, bool parked, uint32_t slot,
+                                            uint32_t ctr, uint32_t rng_s, f3 L) {
+    const ShadeArgs &A = kernargs<ShadeArgs>();
+    const DScene &S = A.S;
+    const RenderParams &P = A.P;
+    const PathState &st = A.st;
+    uint32_t s = 0, ended_job = kInvalid;
+    bool item_end = false, push = valid && !over;
+    f3 accR = {0, 0, 0}, accA = {0, 0, 0}, accN = {0, 0, 0};
+    if (over) {
+        if (Fx::nrc && P.nrc) {
+            const uint32_t tw = st.nrct[slot];
+            if (tw != kInvalid) nrc_emit_training(P, tw & 0x00ffffffu, tw >> 24, L);
+        }
+        const JobView &J = job_of<MULTI>(S, st, slot);
+        accR = ld3(st.accR[slot]) + L / J.total_samples;
+        s = ctr_sample(ctr) + 1u;
+        if (P.aovs) {
+            accA = ld3(st.accA[slot]) + ld3(st.payA[slot]) / J.total_samples;
+            accN = ld3(st.accN[slot]) + ld3(st.payN[slot]) / J.total_samples;
+        }
+        item_end = s == J.batch_size;
+    }
+    /* finished work items take new ones from the wave's item shard */
+    uint32_t ishard = sh, newitem = kInvalid;
+    item_fetch(P.items, P.items_total, P.items_per_shard, P.item_chunk, item_end, ishard, newitem);
+    if (over) {
+        const uint32_t item = st.item[slot];
+        if (item_end) {
+            P.partR[item] = st4(accR, 0.f);
+            if (P.aovs) {
+                P.partA[item] = st4(accA, 0.f);
+                P.partN[item] = st4(accN, 0.f);
+            }
+            if (MULTI) ended_job = st.job[slot]; /* counted below, once per job and wave */
+            st.item[slot] = newitem;
+            if (newitem != kInvalid) {
+                start_item<MULTI, Fx>(S, P, st, slot, newitem);
+                push = true;
+            }
+        } else {
+            const JobView &J = job_of<MULTI>(S, st, slot);
+            const uint32_t litem = item - J.item_begin;
+            const uint32_t pix = litem % J.npix;
+            /* parity: the batch's stream continues; extended: dimension 0 of the next sample */
+            Rng rng = rng_of<Fx>(J, Fx::ext ? 0u : rng_s, litem, s);
+            f3 o, d;
+            camera_ray(J, pix % J.W, pix / J.W, rng, o, d);
+            if (Fx::nrc && P.nrc) nrc_sample_start(P, J, st, slot, litem, s);
+            st.orig[slot] = st4(o, 0.f);
+            st.dir[slot] = st4(d, 0.f);
+            st.beta[slot] = make_float4(1.f, 1.f, 1.f, -1.f); /* w: last scattering pdf, -1 none */
+            st.L[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
+            st.ctr[slot] = ctr_make(s, 0, 0);
+            if (Fx::vol) st.vol[slot] = J.cam_volume >= 0 ? (uint32_t)J.cam_volume : kInvalid;
+            st.rng[slot] = rng.s;
+            st.accR[slot] = st4(accR, 0.f);
+            if (P.aovs) {
+                st.accA[slot] = st4(accA, 0.f);
+                st.accN[slot] = st4(accN, 0.f);
+            }
+            push = true;
+        }
+        st.flags[slot] = 0u;
+    }
+    if (MULTI) job_items_done(S, ended_job);
+    sq_append(P.ext[nxt], sh, push, parked ? slot | kParked : slot);
+}
+
+/* k_shade: one pass over the extension queue's slots: results of the previous bounce's secondary records are added,
+ * the bounce is shaded, and a sample that is over with nothing pending ends here - its radiance goes to the slot's
+ * accumulators, finished work items are written and replaced, the next camera ray is made - before the wave appends
+ * its slots to the next extension queue.  A sample that is over but waits for records of its last bounce or for a
+ * cache query is parked: its queue entry carries kParked and the next pass ends it.
+ *
+ * Bound by its dependent gathers (path state, hit, instance, triangle, light) at 3 waves per SIMD: 145 to 168 VGPRs.
+ * One pass instead of two (a kernel of its own to end samples read the queue, flags and radiance again and wrote them
+ * again), code for the scene's features only (textures that are the default texel cost two dependent loads each) and
+ * arguments read in place took the 1080p field at 64 spp from 152 to 136 ms, the 1080p medium at 32 spp from 202 to
+ * 180 ms and a 64x64 preview from 3.2 to 3.0 ms. */
+template <bool MULTI, class Fx>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(ShadeArgs) {
     __shared__ SQView view;
-    sq_view_load(P.ext[cur], view);
+    const ShadeArgs &A0 = kernargs<ShadeArgs>();
+    const uint32_t cur = A0.cur;
+    const uint32_t nxt = cur ^ 1u;
+    sq_view_load(A0.P.ext[cur], view);
     const uint32_t count = view.pre[kShards];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
+        const ShadeArgs &A = kernargs<ShadeArgs>();
+        const DScene &S = A.S;
+        const RenderParams &P = A.P;
+        const PathState &st = A.st;
         const uint32_t i = base + threadIdx.x;
         const uint32_t sh = shard_of(i & ~63u);
-        uint32_t slot = 0, secmask = 0;
-        bool simple = true;
-        if (i < count) {
-            slot = sq_at(P.ext[cur], view, i);
+        const bool valid = i < count;
+        uint32_t slot = 0, secmask = 0, ctr = 0, rng_s = 0;
+        f3 L = {0, 0, 0};
+        bool simple = true, over = false, parked = false;
+        if (valid) {
+            slot = sq_at(P.ext[cur], view, i) & ~kParked;
             const JobView &J = job_of<MULTI>(S, st, slot);
             simple = !(J.scene_flags & SCENE_HAS_VOLUME_CHANGE);
-            secmask = shade_one(S, J, P, st, slot);
+            const uint32_t flags = st.flags[slot];
+            ctr = st.ctr[slot];
+            L = ld3(st.L[slot]);
+            if (flags & F_SEC0) L = L + ld3(st.sec_c[slot]);
+            if (flags & F_SEC1) L = L + ld3(st.sec_c[st.nsec + slot]);
+            if (flags & F_SEC2) L = L + ld3(st.sec_c[2u * st.nsec + slot]);
+            if (flags & F_DONE) {
+                over = true;
+                rng_s = st.rng[slot];
+            } else {
+                secmask = shade_one<Fx>(S, J, P, st, slot, flags, ctr, L, rng_s, over);
+                if (over && (secmask & (F_SEC0 | F_SEC1 | F_SEC2 | F_NRCQ))) {
+                    over = false;
+                    parked = true;
+                    st.L[slot] = st4(L, 0.f);
+                    st.rng[slot] = rng_s;
+                    st.flags[slot] = F_DONE | (secmask & (F_SEC0 | F_SEC1 | F_SEC2 | F_TPASS));
+                }
+            }
         }
-        /* single-segment shadow rays and 1 - alpha products go to the persistent shadow kernel, the rest
-         * to the general walk */
+        /* single-segment shadow rays and 1 - alpha products go to the persistent shadow walk, the rest to the
+         * general walk */
         const bool to_shd = simple && (secmask & F_SEC0);
         const bool tpass = (secmask & F_TPASS) != 0u;
         uint32_t gen = to_shd ? (secmask & ~F_SEC0) : secmask;
         if (tpass) gen &= ~F_SEC1;
-        sq_append(P.shd, sh, to_shd, slot * 3u);
-        sq_append(P.shd, sh, tpass, slot * 3u + 1u);
+        sq_append(P.shd[nxt], sh, to_shd, slot * 3u);
+        sq_append(P.shd[nxt], sh, tpass, slot * 3u + 1u);
         sq_append(P.sec, sh, (gen & F_SEC0) != 0u, slot * 3u + 0u);
         sq_append(P.sec, sh, (gen & F_SEC1) != 0u, slot * 3u + 1u);
         sq_append(P.sec, sh, (gen & F_SEC2) != 0u, slot * 3u + 2u);
-        if (P.nrc_use) {
+        if (Fx::nrc && P.nrc_use) {
             sq_append(P.nrcq, sh, (secmask & F_NRCQ) != 0u, slot);
             wave_add64(P.stats, S_NRC_FALLBACK, (secmask & F_NRC_FALLBACK) ? 1u : 0u);
         }
+        end_samples<MULTI, Fx>(nxt, sh, valid, over, parked, slot, ctr, rng_s, L);
     }
 }
 
@@ -1442,7 +1627,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
             const uint32_t kind = r % 3u;
             const uint32_t x = sec_ix(st, r);
             const float4 o4 = st.sec_o[x], d4 = st.sec_d[x], c4 = st.sec_c[x];
-            const uint32_t vol = st.sec_v[x];
+            const uint32_t vol = P.media ? (uint32_t)st.sec_v[x] : kInvalid;
             const bool inside = vol != kInvalid;
             const JobView &J = job_of<MULTI>(S, st, r / 3u);
             f3 res = {0, 0, 0};
@@ -1473,7 +1658,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
  * walk with lane refill; opaque scenes stop at the first hit, scenes with
  * transparent materials apply the any-hit product of 1 - alpha. */
 template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
-__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st) {
+__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st, uint32_t cur) {
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
     uint2 *my = stack + threadIdx.x;
     uint32_t nrays = 0;
@@ -1484,7 +1669,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DSc
     uint32_t shard = wave_global_id() % kShards, r = 0;
     for (;;) {
         uint32_t v = 0;
-        if (sq_refill(P.shd, !active, shard, done, v) && !active) {
+        if (sq_refill(P.shd[cur], !active, shard, done, v) && !active) {
             r = v;
             const uint32_t x = sec_ix(st, r);
             const float4 o4 = st.sec_o[x], d4 = st.sec_d[x];
@@ -1516,7 +1701,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DSc
             f3 T = {0, 0, 0};
             if (!shadowed) {
                 T = ALPHA ? mk(ah.T, ah.T, ah.T) : mk(1, 1, 1);
-                const uint32_t vol = st.sec_v[sec_ix(st, r)];
+                const uint32_t vol = P.media ? (uint32_t)st.sec_v[sec_ix(st, r)] : kInvalid;
                 if (vol != kInvalid) {
                     /* raySecondary.rmiss.glsl:24-42 */
                     const float vtend = fminf((float)(uint32_t)job_of<MULTI>(S, st, r / 3u).zfar, w.tmax);
@@ -1534,125 +1719,6 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DSc
     if (COUNT) {
         wave_add64(P.stats, S_NODES_SHD, cnt.nodes);
         wave_add64(P.stats, S_TRIS_SHD, cnt.tris);
-    }
-}
-
-/* ---------------------------------------------------------- k_finish -- */
-/* Completion bookkeeping of a batched render: the lanes of a wave that ended a work item subtract their count from
- * their job's remaining items with one atomic per job present in the wave (same-address atomics serialize in L2,
- * and every item of a large job would otherwise hit the one counter); the lane that takes a counter to zero stamps
- * the job's completion time.  Called in wave-uniform control flow; `job` is kInvalid for lanes that ended nothing. */
-__device__ __forceinline__ void job_items_done(const DScene &S, uint32_t job) {
-    unsigned long long m = __ballot(job != kInvalid);
-    const uint32_t lane = __lane_id();
-    while (m != 0ull) {
-        const int leader = __ffsll((long long)m) - 1;
-        const uint32_t lj = __shfl(job, leader);
-        const unsigned long long same = __ballot(job == lj);
-        if ((int)lane == leader) {
-            const uint32_t n = (uint32_t)__popcll(same);
-            const JobView &J = S.jobs[lj];
-            if (atomicSub(J.remaining, n) == n) *J.done_ticks = wall_clock64();
-        }
-        m &= ~same;
-    }
-}
-
-template <bool MULTI>
-__global__ __launch_bounds__(kBlock) void k_finish(DScene S, RenderParams P, PathState st, uint32_t cur) {
-    __shared__ SQView view;
-    sq_view_load(P.ext[cur], view);
-    sq_reset(P.sec);
-    sq_reset(P.shd);
-    if (P.nrc_use) sq_reset(P.nrcq);
-    const uint32_t count = view.pre[kShards];
-    const uint32_t nxt = cur ^ 1u;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t sh = shard_of(i & ~63u);
-        bool valid = i < count, done = false, item_end = false;
-        uint32_t slot = 0, flags = 0, s = 0, ended_job = kInvalid;
-        f3 L = {0, 0, 0}, accR = {0, 0, 0}, accA = {0, 0, 0}, accN = {0, 0, 0};
-        if (valid) {
-            slot = sq_at(P.ext[cur], view, i);
-            flags = st.flags[slot];
-            L = ld3(st.L[slot]);
-            if (flags & F_SEC0) L = L + ld3(st.sec_c[slot]);
-            if (flags & F_SEC1) L = L + ld3(st.sec_c[st.nsec + slot]);
-            if (flags & F_SEC2) L = L + ld3(st.sec_c[2u * st.nsec + slot]);
-            flags &= ~(F_SEC0 | F_SEC1 | F_SEC2 | F_TPASS);
-            done = (flags & F_DONE) != 0u;
-            if (done && P.nrc) {
-                const uint32_t tw = st.nrct[slot];
-                if (tw != kInvalid) nrc_emit_training(P, tw & 0x00ffffffu, tw >> 24, L);
-            }
-            if (done) {
-                /* end of sample: raygen.rgen.glsl:126-128 */
-                const JobView &J = job_of<MULTI>(S, st, slot);
-                accR = ld3(st.accR[slot]) + L / J.total_samples;
-                s = ctr_sample(st.ctr[slot]) + 1u;
-                if (P.aovs) {
-                    accA = ld3(st.accA[slot]) + ld3(st.payA[slot]) / J.total_samples;
-                    accN = ld3(st.accN[slot]) + ld3(st.payN[slot]) / J.total_samples;
-                }
-                L = {0, 0, 0};
-                item_end = s == J.batch_size;
-            }
-        }
-        /* finished work items take new ones from the wave's item shard */
-        uint32_t ishard = sh, newitem = kInvalid;
-        item_fetch(P.items, P.items_total, P.items_per_shard, P.item_chunk, item_end, ishard, newitem);
-        bool push = valid && !done;
-        if (done) {
-            uint32_t item = st.item[slot];
-            bool alive = true;
-            if (item_end) {
-                P.partR[item] = st4(accR, 0.f);
-                if (P.aovs) {
-                    P.partA[item] = st4(accA, 0.f);
-                    P.partN[item] = st4(accN, 0.f);
-                }
-                if (MULTI) ended_job = st.job[slot]; /* counted below, once per job and wave */
-                item = newitem;
-                st.item[slot] = item;
-                if (item == kInvalid) {
-                    alive = false;
-                } else {
-                    start_item<MULTI>(S, P, st, slot, item);
-                    push = true;
-                }
-            } else {
-                const JobView &J = job_of<MULTI>(S, st, slot);
-                const uint32_t litem = item - J.item_begin;
-                const uint32_t pix = litem % J.npix;
-                /* parity: the batch's stream continues; extended: dimension 0 of the next sample */
-                Rng rng = rng_of(P, J, P.extended ? 0u : st.rng[slot], litem, s);
-                f3 o, d;
-                camera_ray(J, pix % J.W, pix / J.W, rng, o, d);
-                if (P.nrc) nrc_sample_start(P, J, st, slot, litem, s);
-                st.orig[slot] = st4(o, 0.f);
-                st.dir[slot] = st4(d, 0.f);
-                st.beta[slot] = make_float4(1.f, 1.f, 1.f, -1.f); /* w: last scattering pdf, -1 none */
-                st.ctr[slot] = ctr_make(s, 0, 0);
-                st.vol[slot] = J.cam_volume >= 0 ? (uint32_t)J.cam_volume : kInvalid;
-                st.rng[slot] = rng.s;
-                st.accR[slot] = st4(accR, 0.f);
-                if (P.aovs) {
-                    st.accA[slot] = st4(accA, 0.f);
-                    st.accN[slot] = st4(accN, 0.f);
-                }
-                push = true;
-            }
-            (void)alive;
-            flags = 0u;
-        }
-        if (valid) {
-            if (!(done && item_end)) st.L[slot] = st4(L, 0.f);
-            st.flags[slot] = flags;
-        }
-        if (MULTI) job_items_done(S, ended_job);
-        sq_append(P.ext[nxt], sh, push, slot);
     }
 }
 

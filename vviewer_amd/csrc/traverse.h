@@ -71,6 +71,7 @@ struct DScene {
     uint32_t env_type;
     float bg[3];
     float env_intensity;
+    float flat_normal[3]; /* texel of the default normal map */
     JobView job;          /* the render job (single render) */
     const JobView *jobs;  /* the jobs of a batch (batched render), else null */
     uint32_t njobs;

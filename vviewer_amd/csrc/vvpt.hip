@@ -46,6 +46,8 @@ struct SceneHost {
     uint32_t num_instances = 0, num_triangles = 0;
     uint32_t tlas_nodes = 0, blas_nodes = 0, max_depth = 0;
     uint32_t scene_flags = 0;
+    bool textured = false; /* some material binds a texture of its own to a slot other than alpha */
+    bool walks = false; /* some material is transparent (of whatever type) or some instance changes volume */
     uint32_t num_lights = 0;
     uint32_t cube_w = 0;
     uint32_t env_mw = 0, env_mh = 0;
@@ -299,8 +301,8 @@ bool material_is_emissive(const vvpt_material &m) {
            !(std::fabs(m.emissive[0]) <= 0.01f && std::fabs(m.emissive[1]) <= 0.01f && std::fabs(m.emissive[2]) <= 0.01f);
 }
 
-/* Counter block: count and fetch counters of the four queues, then the work-item counters. */
-enum : uint32_t { CB_EXT0 = 0, CB_EXT1 = 2, CB_SEC = 4, CB_SHD = 6, CB_ITEMS = 8, CB_NRCQ = 9, CB_N = 11 };
+/* Counter block: count and fetch counters of the queues, and the work-item counters. */
+enum : uint32_t { CB_EXT0 = 0, CB_EXT1 = 2, CB_SEC = 4, CB_SHD0 = 6, CB_SHD1 = 8, CB_ITEMS = 10, CB_NRCQ = 11, CB_N = 13 };
 constexpr size_t kCounterBytes = (size_t)CB_N * kShards * kPad * sizeof(uint32_t);
 
 /* The environment importance grid of the extended mode: cell weights from the cube map on the device
@@ -740,6 +742,11 @@ static vvpt_status set_scene_parts(vvpt_ctx *c, const vvpt_scene_desc *D, const 
     c->sh.num_instances = D->num_instances;
     c->sh.num_lights = c->sh.parts[0].num_lights;
     c->sh.scene_flags = (any_transparent ? SCENE_HAS_TRANSPARENT : 0u) | (any_volume_change ? SCENE_HAS_VOLUME_CHANGE : 0u);
+    c->sh.walks = any_volume_change;
+    for (const DMaterial &m : mats) {
+        c->sh.walks = c->sh.walks || (m.flags & 2u);
+        for (uint32_t t : {m.tex1[0], m.tex1[1], m.tex1[2], m.tex2[0], m.tex2[1]}) c->sh.textured = c->sh.textured || t >= 3u;
+    }
     c->sh.cube_w = cube_w;
     c->sh.cam = D->camera;
     c->sh.env = D->environment;
@@ -1047,6 +1054,8 @@ vvpt_status make_dscene(vvpt_ctx *c, bool ext, DScene &S) {
     S.bg[1] = sh.env.background[1];
     S.bg[2] = sh.env.background[2];
     S.env_intensity = sh.env.intensity;
+    S.flat_normal[0] = S.flat_normal[1] = 128.0f / 255.0f; /* texel 2: 0xFFFF8080 */
+    S.flat_normal[2] = 1.0f;
     if (ext && sh.env_mw > 0) { /* extended mode: the environment becomes one more light to choose */
         S.env_mw = sh.env_mw;
         S.env_mh = sh.env_mh;
@@ -1149,17 +1158,17 @@ void launch_extend(bool count, dim3 g, hipStream_t s, const DScene &S, const Ren
 }
 template <int STACK, bool MULTI>
 void launch_shadow(bool count, bool alpha, dim3 g, hipStream_t s, const DScene &S, const RenderParams &P,
-                   const PathState &st) {
+                   const PathState &st, uint32_t cur) {
     if (alpha) {
         if (count)
-            hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
+            hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
         else
-            hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
+            hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
     } else {
         if (count)
-            hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
+            hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
         else
-            hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
+            hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
     }
 }
 template <int STACK, bool MULTI>
@@ -1168,6 +1177,32 @@ void launch_secondary(bool count, dim3 g, hipStream_t s, const DScene &S, const 
         hipLaunchKernelGGL((k_secondary<STACK, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
     else
         hipLaunchKernelGGL((k_secondary<STACK, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
+}
+
+/* The features a render's k_shade is compiled for (kernels.h Features). */
+struct RenderFeatures {
+    bool ext, nrc, tex, vol;
+};
+/* Calls f(Features<...>()) for the compiled features that cover fx (a batched render has no radiance cache). */
+template <bool MULTI, class F>
+void with_features(const RenderFeatures &fx, F &&f) {
+    auto tv = [&](auto e, auto n) {
+        constexpr bool E = decltype(e)::value, N = decltype(n)::value;
+        if (fx.tex && fx.vol) f(Features<E, N, true, true>());
+        else if (fx.tex) f(Features<E, N, true, false>());
+        else if (fx.vol) f(Features<E, N, false, true>());
+        else f(Features<E, N, false, false>());
+    };
+    using T = std::true_type;
+    using N = std::false_type;
+    if constexpr (!MULTI) {
+        if (fx.nrc) {
+            tv(T(), T());
+            return;
+        }
+    }
+    if (fx.ext) tv(T(), N());
+    else tv(N(), N());
 }
 
 /* Per-launch hipEvent pairs; launches of kernel k are bracketed by events 2i, 2i+1. */
@@ -1330,7 +1365,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
      * per slot and the shadow queue two (a slot's light-sample segment and the 1 - alpha product in front of the
      * emitter its previous bounce found through a transparent surface can both be queued in one iteration). */
     const uint32_t cap1 = queue_shard_capacity(N);
-    HIP_TRY(c, ensure(c->queues, (size_t)kShards * cap1 * kQueueBlocks * sizeof(uint32_t)));
+    HIP_TRY(c, ensure(c->queues, (size_t)kShards * cap1 * (kQueueBlocks + kShadowRecords) * sizeof(uint32_t)));
     HIP_TRY(c, ensure(c->counters, kCounterBytes));
     HIP_TRY(c, ensure(c->stats, (size_t)kShards * kStatStride * sizeof(unsigned long long)));
     HIP_TRY(c, ensure(c->partials, (size_t)items_max * sizeof(float4) * (aovs ? 3 : 1)));
@@ -1379,7 +1414,8 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     P.ext[0] = mkq(q, kExtendRecords * cap1, CB_EXT0);
     P.ext[1] = mkq(q + (size_t)kShards * cap1, kExtendRecords * cap1, CB_EXT1);
     P.sec = mkq(q + (size_t)2 * kShards * cap1, kSecondaryRecords * cap1, CB_SEC);
-    P.shd = mkq(q + (size_t)(2 + kSecondaryRecords) * kShards * cap1, kShadowRecords * cap1, CB_SHD);
+    P.shd[0] = mkq(q + (size_t)(2 + kSecondaryRecords) * kShards * cap1, kShadowRecords * cap1, CB_SHD0);
+    P.shd[1] = mkq(q + (size_t)kQueueBlocks * kShards * cap1, kShadowRecords * cap1, CB_SHD1);
     if (nrc) {
         /* radiance cache: training blocks of up to min(depth, 16) vertices, 65536 training samples per frame,
          * one query slot per path slot */
@@ -1477,22 +1513,26 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     HIP_TRY(c, hipEventRecord(c->ev0, s));
 
     /* Iteration bound of a launch window (the reference's per-batch fence timeout, :869-876).  A sample lasts at
-     * most depth + 1 iterations (one per bounce, a transparent pass-through or a scattering event included, plus
-     * the walk of its last emitter lookup), so a work item needs at most batch_size (depth + 1) slot-iterations.
-     * While items remain unstarted every slot is busy (k_finish refills a slot in the iteration its item ends),
+     * most depth + 2 iterations (one per bounce, a transparent pass-through or a scattering event included, the walk
+     * of its last emitter lookup, and one more when it ends with results pending), so a work item needs at most
+     * batch_size (depth + 2) slot-iterations.  While items remain unstarted every slot is busy (k_shade refills a slot in the iteration its item ends),
      * so a window of total work T slot-iterations on n slots ends within T / n + one item's length; twice that is
      * the bound.  vvpt_options.max_iterations overrides it. */
     auto window_bound = [&](uint32_t nb_window) -> uint64_t {
-        if (opt.max_iterations) return opt.max_iterations;
+        if (opt.max_iterations) { /* the option allows a sample depth + 1 iterations: the one it may spend parked comes on top */
+            uint32_t depth = 255u;
+            for (const JobView &j : J) depth = std::min(depth, j.depth);
+            return (uint64_t)std::ceil((double)opt.max_iterations * (depth + 2u) / (depth + 1u));
+        }
         double work = 0.0, tail = 0.0;
         if (multi) {
             for (size_t i = 0; i < njobs; ++i) {
-                const double per_item = (double)J[i].batch_size * (J[i].depth + 1u);
+                const double per_item = (double)J[i].batch_size * (J[i].depth + 2u);
                 work += (double)J[i].npix * batches[i] * per_item;
                 if (batches[i]) tail = std::max(tail, per_item);
             }
         } else {
-            tail = (double)J[0].batch_size * (J[0].depth + 1u);
+            tail = (double)J[0].batch_size * (J[0].depth + 2u);
             work = (double)J[0].npix * nb_window * tail;
         }
         const double n = (double)std::max<uint32_t>(1u, std::min<uint64_t>(nslots, multi ? items_max : (uint64_t)nb_window * J[0].npix));
@@ -1506,6 +1546,11 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     uint64_t nrc_trained = 0;
     c->progress.store(0.0f);
     const bool alpha = (S.scene_flags & SCENE_HAS_TRANSPARENT) != 0u;
+    /* k_shade queues general walks only for surfaces that change volume or are transparent */
+    const bool walks = c->sh.walks;
+    RenderFeatures fx = {ext, nrc, c->sh.textured, (S.scene_flags & SCENE_HAS_VOLUME_CHANGE) != 0u};
+    for (const JobView &j : J) fx.vol = fx.vol || j.cam_volume >= 0;
+    P.media = fx.vol ? 1u : 0u;
     /* launch windows: a batched render has one; a single render covers `win` batches per window */
     std::vector<uint32_t> wins;
     if (multi)
@@ -1562,14 +1607,25 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         };
         size_grids();
 
-        /* one wavefront iteration: extend, shade (+ cache queries), shadow, secondary walks, finish / refill */
+        /* one wavefront iteration: the walks of the previous bounce's secondary records, extend, shade (+ cache
+         * queries).  The general walk serves volume boundaries and transparent surfaces only. */
         auto iteration = [&](auto mt, uint32_t cur) -> vvpt_status {
             constexpr bool M = decltype(mt)::value;
+            if (walks) {
+                HIP_TRY(c, kt.begin(VVPT_K_SECONDARY));
+                with_stack(STACK, [&](auto k) { launch_secondary<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st); });
+                HIP_TRY(c, kt.end());
+            }
+            HIP_TRY(c, kt.begin(VVPT_K_SHADOW));
+            with_stack(STACK, [&](auto k) { launch_shadow<decltype(k)::value, M>(count_nodes, alpha, trace_grid, s, S, P, st, cur); });
+            HIP_TRY(c, kt.end());
             HIP_TRY(c, kt.begin(VVPT_K_EXTEND));
             with_stack(STACK, [&](auto k) { launch_extend<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st, cur); });
             HIP_TRY(c, kt.end());
             HIP_TRY(c, kt.begin(VVPT_K_SHADE));
-            hipLaunchKernelGGL(k_shade<M>, g_shade, dim3(kBlock), 0, s, S, P, st, cur);
+            with_features<M>(fx, [&](auto f) {
+                hipLaunchKernelGGL((k_shade<M, decltype(f)>), g_shade, dim3(kBlock), 0, s, ShadeArgs{S, P, st, cur});
+            });
             HIP_TRY(c, kt.end());
             if (P.nrc_use) {
                 /* cache queries of this iteration: gather, infer, add throughput x radiance */
@@ -1581,15 +1637,6 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                 hipLaunchKernelGGL(k_nrc_apply, g_shade, dim3(kBlock), 0, s, P, st);
                 HIP_TRY(c, kt.end());
             }
-            HIP_TRY(c, kt.begin(VVPT_K_SHADOW));
-            with_stack(STACK, [&](auto k) { launch_shadow<decltype(k)::value, M>(count_nodes, alpha, trace_grid, s, S, P, st); });
-            HIP_TRY(c, kt.end());
-            HIP_TRY(c, kt.begin(VVPT_K_SECONDARY));
-            with_stack(STACK, [&](auto k) { launch_secondary<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st); });
-            HIP_TRY(c, kt.end());
-            HIP_TRY(c, kt.begin(VVPT_K_FINISH));
-            hipLaunchKernelGGL(k_finish<M>, g_shade, dim3(kBlock), 0, s, S, P, st, cur);
-            HIP_TRY(c, kt.end());
             return VVPT_OK;
         };
         /* four iterations (the extension queues swap every iteration, so four leave them as they were), eager or
@@ -1605,7 +1652,10 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         auto run_window = [&](auto mt) -> vvpt_status {
             constexpr bool M = decltype(mt)::value;
             uint64_t window_iters = 0;
-            hipLaunchKernelGGL(k_init<M>, dim3((P.nslots + kBlock - 1) / kBlock), dim3(kBlock), 0, s, S, P, st);
+            with_features<M>(fx, [&](auto f) {
+                using Fi = Features<decltype(f)::ext, decltype(f)::nrc, false, true>;
+                hipLaunchKernelGGL((k_init<M, Fi>), dim3((P.nslots + kBlock - 1) / kBlock), dim3(kBlock), 0, s, S, P, st);
+            });
             hipGraphExec_t gx = nullptr;
             if (graph) {
                 hipGraph_t g = nullptr;
