@@ -1,15 +1,19 @@
 /*
  * denoise.hip - edge-avoiding a-trous filter on gfx950 (denoise.h).
  *
- *   k_dn_demod   irradiance = radiance / albedo per channel (albedo below 1e-3 counts as 1), so texture detail
- *                is not blurred; the filter runs on what the albedo multiplies
- *   k_dn_atrous  one level: 5 x 5 taps of the B3-spline kernel (1/16, 1/4, 3/8, 1/4, 1/16) spaced `step`
+ *   k_dn_level   one level: 5 x 5 taps of the B3-spline kernel (1/16, 1/4, 3/8, 1/4, 1/16) spaced `step`
  *                pixels apart, each weighted by exp(-|log(1 + c_q) - log(1 + c_p)|^2 / sigma_c^2) (relative
  *                differences, so an emitter does not bleed into its surroundings; sigma_c halves per level),
  *                max(0, n_p . n_q)^64 and exp(-|a_q - a_p|^2 / sigma_a^2); taps outside the image are skipped
- *                and the weights renormalised
- *   k_dn_remod   radiance = filtered irradiance * albedo, alpha 1
- * Every pixel is one thread; each level reads its 25 taps from L2 (a 1080p level is 2M x 25 float4 reads).
+ *                and the weights renormalised.  The first level divides the radiance by the albedo per channel
+ *                (albedo below 1e-3 counts as 1), so texture detail is not blurred and the filter runs on what the
+ *                albedo multiplies; the last multiplies it back, alpha 1.
+ *
+ * A block filters 16 x 16 pixels of one residue class (x mod step, y mod step), whose taps are each other's neighbours:
+ * the 20 x 20 pixels they need are read, their logarithms taken and their normals decoded once, into LDS, instead of 25
+ * times per pixel.  The step's step^2 classes of one image region are consecutive blocks of one die, so that the
+ * interleaved lines they read are shared in its L2.  Bound by instruction issue (25 taps of about 45 instructions per
+ * pixel).  1920 x 1080: 75 to 95 us a level instead of 571, the whole filter 0.375 ms instead of 2.45.
  */
 #include "denoise.h"
 
@@ -43,79 +47,109 @@ __device__ __forceinline__ bool dn_normal(float4 e, float3 &n) {
     return true;
 }
 
-__global__ void k_dn_demod(const float4 *rad, const float4 *alb, uint32_t n, float4 *irr) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 r = rad[i], a = alb[i];
-    irr[i] = make_float4(r.x / dn_demod(a.x), r.y / dn_demod(a.y), r.z / dn_demod(a.z), 0.0f);
-}
+constexpr int kDnTile = 16, kDnHalo = kDnTile + 4; /* outputs and staged pixels of a block, per axis */
 
-__global__ void k_dn_atrous(const float4 *src, float4 *dst, const float4 *alb, const float4 *nrm, uint32_t W,
-                            uint32_t H, int step, float inv_sc2) {
-    const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y;
-    if (x >= W || y >= H) return;
+template <bool FIRST, bool LAST>
+__global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *src, float4 *dst, const float4 *alb,
+                                                                const float4 *nrm, uint32_t W, uint32_t H, int step,
+                                                                uint32_t tiles_x, uint32_t nblocks, float inv_sc2) {
+    /* a staged pixel: (c, t.x), (t.y, t.z, a.x, a.y), (a.z, n); n = 0 where the pixel saw no surface, and an albedo no
+     * image holds outside the image, whose weight underflows to 0 */
+    __shared__ float4 tile[3][kDnHalo * kDnHalo];
+    /* the blocks of one die (block % 8) take consecutive (tile, y class, x class) triples */
+    const uint32_t per = (nblocks + 7u) / 8u, lin = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if (lin >= nblocks) return;
+    const uint32_t us = (uint32_t)step, rx = lin % us, ry = lin / us % us, tl = lin / (us * us);
+    const int tx = (int)(tl % tiles_x) * kDnTile, ty = (int)(tl / tiles_x) * kDnTile; /* in pixels of the class */
+    for (int k = threadIdx.x; k < kDnHalo * kDnHalo; k += kDnTile * kDnTile) {
+        const int qx = (tx + k % kDnHalo - 2) * step + (int)rx, qy = (ty + k / kDnHalo - 2) * step + (int)ry;
+        float4 c = make_float4(0.f, 0.f, 0.f, 0.f), t = c, a = make_float4(1e15f, 0.f, 0.f, 0.f);
+        float3 n = make_float3(0.f, 0.f, 0.f);
+        if (qx >= 0 && qx < (int)W && qy >= 0 && qy < (int)H) {
+            const size_t q = (size_t)qy * W + qx;
+            c = src[q];
+            a = alb[q];
+            if (FIRST) c = make_float4(c.x / dn_demod(a.x), c.y / dn_demod(a.y), c.z / dn_demod(a.z), 0.0f);
+            t = dn_compress(c);
+            if (!dn_normal(nrm[q], n)) n = make_float3(0.f, 0.f, 0.f);
+        }
+        tile[0][k] = make_float4(c.x, c.y, c.z, t.x);
+        tile[1][k] = make_float4(t.y, t.z, a.x, a.y);
+        tile[2][k] = make_float4(a.z, n.x, n.y, n.z);
+    }
+    __syncthreads();
+    const int lx = threadIdx.x % kDnTile, ly = threadIdx.x / kDnTile;
+    const int x = (tx + lx) * step + (int)rx, y = (ty + ly) * step + (int)ry;
+    if (x >= (int)W || y >= (int)H) return;
     const float h[5] = {1.0f / 16.0f, 1.0f / 4.0f, 3.0f / 8.0f, 1.0f / 4.0f, 1.0f / 16.0f};
-    const size_t p = (size_t)y * W + x;
-    const float4 cp = src[p], tp = dn_compress(cp), ap = alb[p];
-    float3 np;
-    const bool sp = dn_normal(nrm[p], np);
+    const int centre = (ly + 2) * kDnHalo + lx + 2;
+    const float4 p0 = tile[0][centre], p1 = tile[1][centre], p2 = tile[2][centre];
+    const bool sp = p2.y != 0.0f || p2.z != 0.0f || p2.w != 0.0f;
     const float inv_sa2 = 1.0f / (kDenoiseSigmaAlbedo * kDenoiseSigmaAlbedo);
     float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float wsum = 0.0f;
+#pragma unroll 1 /* a row's taps in flight: all 25 unrolled hold 258 registers */
     for (int j = 0; j < 5; ++j) {
-        const int qy = (int)y + (j - 2) * step;
-        if (qy < 0 || qy >= (int)H) continue;
+        const float hj = j == 2 ? 3.0f / 8.0f : ((j & 1) ? 1.0f / 4.0f : 1.0f / 16.0f);
+#pragma unroll
         for (int i = 0; i < 5; ++i) {
-            const int qx = (int)x + (i - 2) * step;
-            if (qx < 0 || qx >= (int)W) continue;
-            const size_t q = (size_t)qy * W + qx;
-            const float4 cq = src[q], tq = dn_compress(cq), aq = alb[q];
-            float3 nq;
-            const bool sq = dn_normal(nrm[q], nq);
-            const float dc = (tq.x - tp.x) * (tq.x - tp.x) + (tq.y - tp.y) * (tq.y - tp.y) + (tq.z - tp.z) * (tq.z - tp.z);
-            const float da = (aq.x - ap.x) * (aq.x - ap.x) + (aq.y - ap.y) * (aq.y - ap.y) + (aq.z - ap.z) * (aq.z - ap.z);
+            const int k = (ly + j) * kDnHalo + lx + i;
+            const float4 q0 = tile[0][k], q1 = tile[1][k], q2 = tile[2][k];
+            const float dx = q0.w - p0.w, dy = q1.x - p1.x, dz = q1.y - p1.y;
+            const float ax = q1.z - p1.z, ay = q1.w - p1.w, az = q2.x - p2.x;
+            const float dc = dx * dx + dy * dy + dz * dz, da = ax * ax + ay * ay + az * az;
             float wn;
-            if (sp && sq)
-                wn = __powf(fmaxf(np.x * nq.x + np.y * nq.y + np.z * nq.z, 0.0f), kDenoiseNormalPower);
-            else
-                wn = (sp == sq) ? 1.0f : 0.0f;
-            const float w = h[i] * h[j] * __expf(-dc * inv_sc2 - da * inv_sa2) * wn;
-            sum.x += w * cq.x;
-            sum.y += w * cq.y;
-            sum.z += w * cq.z;
+            if (sp) { /* 0 against a pixel without a surface */
+                wn = fmaxf(p2.y * q2.y + p2.z * q2.z + p2.w * q2.w, 0.0f);
+                static_assert(kDenoiseNormalPower == 64.0f, "six squarings");
+#pragma unroll
+                for (int e = 0; e < 6; ++e) wn *= wn;
+            } else {
+                wn = (q2.y != 0.0f || q2.z != 0.0f || q2.w != 0.0f) ? 0.0f : 1.0f;
+            }
+            const float w = h[i] * hj * __expf(-dc * inv_sc2 - da * inv_sa2) * wn;
+            sum.x += w * q0.x;
+            sum.y += w * q0.y;
+            sum.z += w * q0.z;
             wsum += w;
         }
     }
     /* the centre tap has weight h2 * h2 > 0, so wsum > 0 */
     const float r = 1.0f / wsum;
-    dst[p] = make_float4(sum.x * r, sum.y * r, sum.z * r, 0.0f);
-}
-
-__global__ void k_dn_remod(const float4 *irr, const float4 *alb, uint32_t n, float4 *out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 c = irr[i], a = alb[i];
-    out[i] = make_float4(c.x * dn_demod(a.x), c.y * dn_demod(a.y), c.z * dn_demod(a.z), 1.0f);
+    const size_t p = (size_t)y * W + x;
+    if (LAST)
+        dst[p] = make_float4(sum.x * r * dn_demod(p1.z), sum.y * r * dn_demod(p1.w), sum.z * r * dn_demod(p2.x), 1.0f);
+    else
+        dst[p] = make_float4(sum.x * r, sum.y * r, sum.z * r, 0.0f);
 }
 
 }  // namespace
 
 std::string denoise_device(const float *radiance, const float *albedo, const float *normal, uint32_t W, uint32_t H,
                            float *out, float *tmp, hipStream_t s) {
-    const uint32_t n = W * H;
-    float4 *a = (float4 *)tmp, *b = a + n;
-    const float4 *alb = (const float4 *)albedo, *nrm = (const float4 *)normal;
-    hipLaunchKernelGGL(k_dn_demod, dim3((n + 255) / 256), dim3(256), 0, s, (const float4 *)radiance, alb, n, a);
-    const dim3 blk(16, 16), grid((W + 15) / 16, (H + 15) / 16);
+    /* every level reads what the one before it wrote, the first the radiance; only the last writes out, which may be the
+     * radiance itself */
+    float4 *img[2] = {(float4 *)tmp, (float4 *)tmp + (size_t)W * H};
+    const float4 *src = (const float4 *)radiance, *alb = (const float4 *)albedo, *nrm = (const float4 *)normal;
     float sc = kDenoiseSigmaColor;
+    static_assert(kDenoiseLevels >= 2, "the first and the last level are different launches");
     for (int l = 0; l < kDenoiseLevels; ++l) {
-        hipLaunchKernelGGL(k_dn_atrous, grid, blk, 0, s, a, b, alb, nrm, W, H, 1 << l, 1.0f / (sc * sc));
-        float4 *t = a;
-        a = b;
-        b = t;
+        const uint32_t step = 1u << l;
+        const uint32_t tiles_x = ((W + step - 1) / step + kDnTile - 1) / kDnTile;
+        const uint32_t tiles_y = ((H + step - 1) / step + kDnTile - 1) / kDnTile;
+        const uint32_t nblocks = tiles_x * tiles_y * step * step;
+        const dim3 grid((nblocks + 7u) / 8u * 8u), blk(kDnTile * kDnTile);
+        float4 *dst = l + 1 == kDenoiseLevels ? (float4 *)out : img[l & 1];
+        const float inv_sc2 = 1.0f / (sc * sc);
+        if (l == 0)
+            hipLaunchKernelGGL((k_dn_level<true, false>), grid, blk, 0, s, src, dst, alb, nrm, W, H, (int)step, tiles_x, nblocks, inv_sc2);
+        else if (l + 1 < kDenoiseLevels)
+            hipLaunchKernelGGL((k_dn_level<false, false>), grid, blk, 0, s, src, dst, alb, nrm, W, H, (int)step, tiles_x, nblocks, inv_sc2);
+        else
+            hipLaunchKernelGGL((k_dn_level<false, true>), grid, blk, 0, s, src, dst, alb, nrm, W, H, (int)step, tiles_x, nblocks, inv_sc2);
+        src = dst;
         sc *= 0.5f;
     }
-    hipLaunchKernelGGL(k_dn_remod, dim3((n + 255) / 256), dim3(256), 0, s, a, alb, n, (float4 *)out);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? std::string() : std::string(hipGetErrorString(e));
 }
@@ -144,7 +178,7 @@ std::string denoise_device_noalloc(const float *radiance, const float *albedo, c
         if (device >= 0 && (size_t)device < g_scratch_ptr.size()) tmp = g_scratch_ptr[device];
     }
     if (!tmp) return "no scratch address on this device";
-    /* demod writes every pixel of the first image and each level every pixel of the next before they are read:
+    /* the first level writes every pixel of the first image and each level every pixel of the next before they are read:
      * nothing in the scratch needs to start at zero, and what a previous call left there is never read */
     return denoise_device(radiance, albedo, normal, W, H, out, (float *)tmp, stream);
 }
