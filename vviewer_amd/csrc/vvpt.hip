@@ -1771,11 +1771,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                         std::this_thread::sleep_for(std::chrono::microseconds(20));
                 }
             }
-            if (gx) {
-                /* iterations beyond the last one may still be queued: their arguments live in the executable graph */
-                (void)hipStreamSynchronize(s);
-                (void)hipGraphExecDestroy(gx);
-            }
+            if (gx) (void)hipGraphExecDestroy(gx);
             return v;
         };
         const vvpt_status vw = multi ? run_window(std::true_type()) : run_window(std::false_type());
