@@ -143,8 +143,6 @@ struct RenderParams {
     uint32_t items_per_shard;
     uint32_t item_chunk; /* 0: contiguous item shards; else chunks of this many items dealt round-robin */
     unsigned long long *stats; /* kShards * kStatStride */
-    uint32_t *tick;                    /* iterations begun in this render */
-    unsigned long long *host_progress; /* pinned host memory: [0] iteration << 32 | live slots, [1] items started */
     float4 *partR, *partA, *partN;
     /* radiance cache */
     uint32_t nrc;              /* the cache is trained on this render's paths */
@@ -1737,43 +1735,6 @@ __device__ __forceinline__ void reset_next_queues(const RenderParams &P, uint32_
     if (P.nrc_use) sq_reset(P.nrcq);
 }
 
-/* Tells the host, at the start of an iteration's path walks, which iteration begins, how many slots are live in it and
- * how many work items have been started, so that the host can keep launches queued without draining the stream to
- * look (a copy and a wait every four iterations left the chip idle for 50 us each).  Block 0's first wave. */
-__device__ __forceinline__ void report_progress(const RenderParams &P, uint32_t cur) {
-    if (blockIdx.x != 0u || threadIdx.x >= kShards) return;
-    const uint32_t s = threadIdx.x, per = P.items_per_shard;
-    uint32_t live = *sq_count(P.ext[cur], s);
-    uint32_t started = min(P.items[s * kPad], per) - (per - item_shard_size(P.items_total, per, P.item_chunk, s));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        live += __shfl_xor(live, o);
-        started += __shfl_xor(started, o);
-    }
-    if (s == 0u) {
-        const uint32_t n = *P.tick + 1u;
-        *P.tick = n;
-        __hip_atomic_store(P.host_progress + 1, (unsigned long long)started, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(P.host_progress, (unsigned long long)n << 32 | live, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-}
-
-/* Counters of a launch window: every queue counter zero, item shard s at per - size_s (queue.h item_fetch).  The first
- * window of a render also clears its statistics and the iteration count. */
-__global__ __launch_bounds__(kBlock) void k_window_init(RenderParams P, uint32_t *counters, uint32_t n, uint32_t first) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const uint32_t k = i - (uint32_t)(P.items - counters); /* wraps below the item counters */
-        counters[i] = k < kShards * kPad && k % kPad == 0u
-                          ? P.items_per_shard - item_shard_size(P.items_total, P.items_per_shard, P.item_chunk, k / kPad)
-                          : 0u;
-    }
-    if (first) {
-        if (i < kShards * kStatStride) P.stats[i] = 0ull;
-        if (i == 0u) *P.tick = 0u;
-    }
-}
-
 /* The single-segment shadow rays of the previous bounce (kTraceShadows) and the path rays of this one (kTracePaths).
  * Bound by instruction issue and load latency (the geometry is cache-resident): at least 5 waves per SIMD (at most 102
  * VGPRs; 4 otherwise) where the LDS stack allows it (STACK <= 16); 6 waves would spill registers to scratch, and so
@@ -1789,7 +1750,6 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(Loo
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock];
     const LoopArgs &A = kernargs<LoopArgs>();
     reset_next_queues(A.P, A.cur);
-    report_progress(A.P, A.cur);
     trace_paths<STACK, COUNT, MULTI, 1>(stack + threadIdx.x, A.cur);
 }
 
@@ -1804,7 +1764,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace8(LoopArgs) {
     const LoopArgs &A = kernargs<LoopArgs>();
     const uint32_t cur = A.cur, phases = A.phases;
     reset_next_queues(A.P, cur);
-    if (phases & kTracePaths) report_progress(A.P, cur);
     bool shadows = (blockIdx.x & 1u) == 0u;
     for (int k = 0; k < 2; ++k) {
         if (shadows) {

@@ -18,7 +18,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -93,8 +92,6 @@ struct vvpt_ctx {
     /* render buffers (grown on demand) */
     DevBuf state, queues, counters, stats, partials, outputs;
     uint32_t *h_counters = nullptr; /* pinned copy of the counter block */
-    unsigned long long *h_progress = nullptr; /* pinned: what the loop's kernels report (report_progress) */
-    unsigned long long *h_stats = nullptr;    /* pinned copy of the statistics */
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::vector<hipEvent_t> kev; /* per-launch timing events (VVPT_FLAG_KERNEL_TIMING) */
     uint32_t builder = VVPT_BUILDER_SAH;
@@ -307,7 +304,6 @@ bool material_is_emissive(const vvpt_material &m) {
 /* Counter block: count and fetch counters of the queues, and the work-item counters. */
 enum : uint32_t { CB_EXT0 = 0, CB_EXT1 = 2, CB_SEC = 4, CB_SHD0 = 6, CB_SHD1 = 8, CB_ITEMS = 10, CB_NRCQ = 11, CB_N = 13 };
 constexpr size_t kCounterBytes = (size_t)CB_N * kShards * kPad * sizeof(uint32_t);
-constexpr size_t kStatBytes = (size_t)kShards * kStatStride * sizeof(unsigned long long);
 
 /* The environment importance grid of the extended mode: cell weights from the cube map on the device
  * (k_env_importance), a floor of 1 % of the mean radiance so that every direction keeps some density, and the
@@ -408,8 +404,6 @@ vvpt_status vvpt_create(vvpt_ctx **out, int hip_device) {
     c->cus = (uint32_t)prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipHostMalloc((void **)&c->h_counters, kCounterBytes, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&c->h_progress, 64, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&c->h_stats, kStatBytes, hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         vvpt_destroy(c);
         return VVPT_DEVICE_LOST;
@@ -438,8 +432,6 @@ void vvpt_destroy(vvpt_ctx *c) {
                       &c->queues, &c->counters, &c->stats, &c->partials, &c->outputs};
     for (DevBuf *b : bufs) release(*b);
     if (c->h_counters) (void)hipHostFree(c->h_counters);
-    if (c->h_progress) (void)hipHostFree(c->h_progress);
-    if (c->h_stats) (void)hipHostFree(c->h_stats);
     for (hipEvent_t e : c->kev) (void)hipEventDestroy(e);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -1251,10 +1243,6 @@ struct JobSpec {
     float *rad, *alb, *nrm;
 };
 
-/* Iterations the host launches beyond the one that has begun: enough to keep the stream fed while the host sees a
- * report and launches the next, and few, because those beyond the last one run empty. */
-constexpr uint64_t kIterationsAhead = 2;
-
 /* Launches with at most this many live slots per compute unit walk each ray with eight lanes (traverse.h trav_step):
  * at 10,240 path rays and as many shadow rays they make 2,560 waves, 2.5 for each SIMD.  A 64x64 Cornell box (16,384 slots, falling)
  * took 2.12 / 2.03 / 2.29 ms with the line at 20 / 40 / 80 and 2.3 without group walks, the 640x360 field of 10,000
@@ -1382,8 +1370,8 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
      * emitter its previous bounce found through a transparent surface can both be queued in one iteration). */
     const uint32_t cap1 = queue_shard_capacity(N);
     HIP_TRY(c, ensure(c->queues, (size_t)kShards * cap1 * (kQueueBlocks + kShadowRecords) * sizeof(uint32_t)));
-    HIP_TRY(c, ensure(c->counters, kCounterBytes + 256)); /* and the iteration count */
-    HIP_TRY(c, ensure(c->stats, kStatBytes));
+    HIP_TRY(c, ensure(c->counters, kCounterBytes));
+    HIP_TRY(c, ensure(c->stats, (size_t)kShards * kStatStride * sizeof(unsigned long long)));
     HIP_TRY(c, ensure(c->partials, (size_t)items_max * sizeof(float4) * (aovs ? 3 : 1)));
     char *sb = (char *)c->state.p;
     PathState st;
@@ -1497,9 +1485,6 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     }
     P.items = cb + (size_t)CB_ITEMS * kShards * kPad;
     P.stats = (unsigned long long *)c->stats.p;
-    P.tick = (uint32_t *)((char *)c->counters.p + kCounterBytes);
-    P.host_progress = c->h_progress;
-    c->h_progress[0] = c->h_progress[1] = 0ull; /* no kernel of this context runs here */
     float4 *pp = (float4 *)c->partials.p;
     P.partR = pp;
     P.partA = aovs ? pp + items_max : nullptr;
@@ -1528,6 +1513,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         S.njobs = (uint32_t)nj;
     }
 
+    HIP_TRY(c, hipMemsetAsync(c->stats.p, 0, (size_t)kShards * kStatStride * sizeof(unsigned long long), s));
     HIP_TRY(c, hipEventRecord(c->ev0, s));
 
     /* Iteration bound of a launch window (the reference's per-batch fence timeout, :869-876).  A sample lasts at
@@ -1596,9 +1582,12 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         P.item_chunk = multi ? kItemChunk : 0u;
         P.items_per_shard = multi ? item_shard_size(P.items_total, 0u, P.item_chunk, 0u)
                                   : (P.items_total + kShards - 1) / kShards;
-        constexpr uint32_t kCounters = (uint32_t)(kCounterBytes / sizeof(uint32_t));
-        hipLaunchKernelGGL(k_window_init, dim3((kCounters + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, cb, kCounters,
-                           w == 0 ? 1u : 0u);
+        /* every counter zero; item shard s starts at per - size_s (queue.h item_fetch) */
+        std::vector<uint32_t> init(kCounterBytes / 4, 0u);
+        for (uint32_t sh = 0; sh < kShards; ++sh)
+            init[(size_t)CB_ITEMS * kShards * kPad + sh * kPad] =
+                P.items_per_shard - item_shard_size(P.items_total, P.items_per_shard, P.item_chunk, sh);
+        HIP_TRY(c, hipMemcpyAsync(cb, init.data(), kCounterBytes, hipMemcpyHostToDevice, s));
         if (nrc) {
             HIP_TRY(c, hipMemsetAsync(P.nrc_ctr, 0, 256, s));
             P.nrc_use = b0 > 0 ? 1u : 0u; /* the first frame only trains */
@@ -1608,6 +1597,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
             if (last) P.nrc_thresh = 0u;
             P.nrc = (P.nrc_use || !last) ? 1u : 0u;
         }
+        HIP_TRY(c, hipStreamSynchronize(s));
         if (multi) hipLaunchKernelGGL(k_clock_stamp, dim3(1), dim3(64), 0, s, d_ticks + djobs.size());
         /* Slots that can still hold a path: all of them at first, then what the last counter readback found (a slot
          * without a work item never gets one again, so the count only falls).  Launches are sized to it: a lane per
@@ -1699,86 +1689,51 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                 HIP_TRY(c, ei);
             }
             vvpt_status v = VVPT_OK;
-            const uint64_t before = iterations; /* of earlier windows */
-            const uint32_t step = gx ? 4u : 1u;
-            using clock = std::chrono::steady_clock;
-            clock::time_point since = clock::now();
-            uint64_t seen = before;
-            for (uint32_t spins = 0;; ++spins) {
-                /* what the kernels reported last: iteration `tag` (counted over the render) began with `act` live slots */
-                const unsigned long long rep = __atomic_load_n(&c->h_progress[0], __ATOMIC_ACQUIRE);
-                const uint64_t tag = rep >> 32;
-                const uint32_t act = (uint32_t)rep;
-                if (tag > seen) {
-                    seen = tag;
-                    since = clock::now();
-                    const uint64_t started = __atomic_load_n(&c->h_progress[1], __ATOMIC_RELAXED);
-                    const uint64_t done = items_done_before + (started > act ? started - act : 0);
-                    c->progress.store((float)((double)std::min<uint64_t>(done, total_items) / (double)total_items));
-                    if (act == 0u) break;
-                    if (!gx) { /* a captured graph keeps its grids */
-                        live = std::min(act, P.nslots);
-                        size_grids();
+            for (;;) {
+                if (gx) {
+                    const hipError_t e = hipGraphLaunch(gx, s);
+                    if (e != hipSuccess) {
+                        v = set_err(c, VVPT_DEVICE_LOST, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
+                        break;
                     }
+                } else {
+                    v = group(mt);
+                    if (v != VVPT_OK) break;
                 }
-                if (iterations - seen < kIterationsAhead && window_iters < max_iters) {
-                    if (gx) {
-                        const hipError_t e = hipGraphLaunch(gx, s);
-                        if (e != hipSuccess) {
-                            v = set_err(c, VVPT_DEVICE_LOST, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
-                            break;
-                        }
-                    } else {
-                        v = iteration(mt, (uint32_t)(window_iters & 1u));
-                        if (v != VVPT_OK) break;
-                    }
-                    iterations += step;
-                    window_iters += step;
-                    spins = 0;
-                    continue;
+                iterations += 4;
+                window_iters += 4;
+                hipError_t e = hipMemcpyAsync(c->h_counters, cb, kCounterBytes, hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipStreamSynchronize(s);
+                if (e != hipSuccess) {
+                    v = set_err(c, VVPT_DEVICE_LOST, std::string("counter readback: ") + hipGetErrorString(e));
+                    break;
                 }
-                __builtin_ia32_pause();
-                const bool last = iterations == seen; /* everything launched has begun, and the bound stops more */
-                if (last || spins >= 4096u) {
-                    spins = 0;
-                    const hipError_t e = last ? hipStreamSynchronize(s) : hipStreamQuery(s);
-                    if (e != hipSuccess && e != hipErrorNotReady) {
-                        v = set_err(c, VVPT_DEVICE_LOST, std::string("render loop: ") + hipGetErrorString(e));
-                        break;
-                    }
-                    if (last) {
-                        /* the bound's iterations are over: are any slots left? */
-                        const hipError_t ec = hipMemcpy(c->h_counters, cb, kCounterBytes, hipMemcpyDeviceToHost);
-                        if (ec != hipSuccess) {
-                            v = set_err(c, VVPT_DEVICE_LOST, std::string("counter readback: ") + hipGetErrorString(ec));
-                            break;
-                        }
-                        const uint32_t *extc =
-                            c->h_counters + (size_t)((window_iters & 1u) ? CB_EXT1 : CB_EXT0) * kShards * kPad;
-                        uint64_t active = 0;
-                        for (uint32_t sh = 0; sh < kShards; ++sh) active += extc[sh * kPad];
-                        if (active != 0u)
-                            v = set_err(c, VVPT_TIMEOUT, "render did not finish within " + std::to_string(max_iters) +
-                                                             " wavefront iterations");
-                        break;
-                    }
-                    if (e == hipSuccess && (__atomic_load_n(&c->h_progress[0], __ATOMIC_ACQUIRE) >> 32) < iterations) {
-                        v = set_err(c, VVPT_DEVICE_LOST, "render loop: the launched iterations reported no progress");
-                        break;
-                    }
-                    /* long iterations: leave the core to others */
-                    if (clock::now() - since > std::chrono::microseconds(200))
-                        std::this_thread::sleep_for(std::chrono::microseconds(20));
+                uint64_t active = 0, started = 0;
+                const uint32_t *extc = c->h_counters + (size_t)CB_EXT0 * kShards * kPad;
+                const uint32_t *itc = c->h_counters + (size_t)CB_ITEMS * kShards * kPad;
+                for (uint32_t sh = 0; sh < kShards; ++sh) {
+                    active += extc[sh * kPad];
+                    const uint32_t skip = P.items_per_shard - item_shard_size(P.items_total, P.items_per_shard, P.item_chunk, sh);
+                    started += std::min<uint32_t>(itc[sh * kPad], P.items_per_shard) - skip;
+                }
+                const uint64_t done = items_done_before + (started > active ? started - active : 0);
+                c->progress.store((float)((double)done / (double)total_items));
+                if (active == 0u) break;
+                if (!gx) { /* a captured graph keeps its grids */
+                    live = (uint32_t)std::min<uint64_t>(active, P.nslots);
+                    size_grids();
+                }
+                if (window_iters >= max_iters) {
+                    v = set_err(c, VVPT_TIMEOUT, "render did not finish within " + std::to_string(max_iters) +
+                                                     " wavefront iterations");
+                    break;
                 }
             }
             if (gx) (void)hipGraphExecDestroy(gx);
             return v;
         };
         const vvpt_status vw = multi ? run_window(std::true_type()) : run_window(std::false_type());
-        if (vw != VVPT_OK) {
-            (void)hipStreamSynchronize(s); /* what was launched ends before the caller goes on */
-            return vw;
-        }
+        if (vw != VVPT_OK) return vw;
         if (!multi) {
             hipLaunchKernelGGL(k_resolve, dim3((J[0].npix + kBlock - 1) / kBlock), dim3(kBlock), 0, s, P, S.job, nb,
                                w == 0 ? 1u : 0u, (float4 *)jobs[0].rad, (float4 *)jobs[0].alb, (float4 *)jobs[0].nrm);
@@ -1823,7 +1778,6 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
         }
     }
     HIP_TRY(c, hipEventRecord(c->ev1, s));
-    if (stats) HIP_TRY(c, hipMemcpyAsync(c->h_stats, c->stats.p, kStatBytes, hipMemcpyDeviceToHost, s));
     HIP_TRY(c, hipGetLastError());
     HIP_TRY(c, hipStreamSynchronize(s));
     c->progress.store(1.0f);
@@ -1841,7 +1795,8 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
             }
     }
     if (stats) {
-        const unsigned long long *hsh = c->h_stats;
+        std::vector<unsigned long long> hsh((size_t)kShards * kStatStride);
+        HIP_TRY(c, hipMemcpy(hsh.data(), c->stats.p, hsh.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
         unsigned long long hs[S_NSTATS] = {0};
         for (uint32_t sh = 0; sh < kShards; ++sh)
             for (uint32_t k = 0; k < S_NSTATS; ++k) hs[k] += hsh[(size_t)sh * kStatStride + k];
