@@ -12,9 +12,9 @@
  *   k_secondary  shadow segments and emitter-lookup walks of the previous bounce that need the general walk (any-hit
  *                logic applied closest-first)
  *   k_shadow     single-segment shadow rays of the previous bounce
- *   k_extend     closest-hit query of each slot's ray; when the previous bounce asked for a BSDF-direction emitter
- *                lookup (next_event_estimation.glsl) the same walk also answers it (MODE_CLOSEST2)
- *   k_trace8     both of them in launches with few rays
+ *   k_extend     closest-hit query of each slot's ray; when the previous bounce
+ *                asked for a BSDF-direction emitter lookup (next_event_estimation.glsl)
+ *                the same walk also answers it (MODE_CLOSEST2)
  *   k_shade      adds the previous bounce's secondary results in a fixed order, then one bounce of the closest-hit /
  *                miss shaders; light sampling and emitter lookups that need their own walk become records in a
  *                shadow or secondary queue; samples that end are accumulated, finished work items written and
@@ -35,7 +35,10 @@
 namespace vvpt {
 
 constexpr int kTraceBlock = 128;
-/* Occupancy of k_extend and k_shadow (see there). */
+/* k_extend and k_shadow: at least 5 waves per SIMD (at most 102 VGPRs; 4 otherwise) where the LDS stack allows it
+ * (STACK <= 16).  Their walks wait on dependent node loads, so resident waves hide latency (k_shadow 116 -> 107 ms
+ * per 1080p frame at 64 spp; k_extend 67.3 -> 62.4 ms once its world ray and saved TLAS position moved to LDS and it
+ * fitted in 92 VGPRs without spilling); 6 waves would spill registers to scratch. */
 #define VVPT_TRACE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(STACK <= 16 ? 5 : 1, 8)))
 constexpr int kBlock = 256;
 
@@ -114,7 +117,7 @@ struct PathState {
     StreamArray<uint32_t> item, rng, ctr, vol, flags;
     StreamArray<uint32_t> job; /* batched render: the slot's job */
     StreamArray<float4> orig, dir, beta, nee, L, accR, accA, accN, payA, payN;
-    /* The walk's answer, one 64-byte record per slot (4 s .. 4 s + 3), so that a finished walk writes whole 32-byte
+    /* k_extend's answer, one 64-byte record per slot (4 s .. 4 s + 3), so that a finished walk writes whole 32-byte
      * sectors of one line instead of parts of five arrays: [0] the path hit (t, u, v, prim); [1] its instance, the
      * emitter lookup's instance and the nearest candidate that lookup passed; [2] the lookup's hit (t, u, v, prim)
      * and [3] zero, written only with a lookup */
@@ -687,6 +690,59 @@ __global__ __launch_bounds__(kBlock) void k_init(DScene S, RenderParams P, PathS
     sq_append(P.ext[0], shard_of(i0), active, i);
 }
 
+/* ---------------------------------------------------------- k_extend -- */
+template <int STACK, bool COUNT, bool MULTI>
+__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(DScene S, RenderParams P, PathState st, uint32_t cur) {
+    __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
+    uint2 *my = stack + threadIdx.x;
+    /* the queues that this iteration's k_shade fills; their last consumers ran before this kernel */
+    sq_reset(P.ext[cur ^ 1u]);
+    sq_reset(P.shd[cur ^ 1u]);
+    sq_reset(P.sec);
+    if (P.nrc_use) sq_reset(P.nrcq);
+    const SQueue &Q = P.ext[cur];
+    uint32_t nrays = 0;
+    TraceCount cnt = {0, 0};
+    Trav w;
+    bool active = false, done = false, nee = false;
+    uint32_t shard = wave_global_id() % kShards, slot = 0;
+    for (;;) {
+        uint32_t v = 0;
+        if (sq_refill(Q, !active, shard, done, v) && !active && !(v & kParked)) {
+            slot = v;
+            const f3 O = ld3(st.orig[slot]), D = ld3(st.dir[slot]);
+            const uint32_t fl = st.flags[slot];
+            nee = (fl & F_NEE) != 0u;
+            /* with a pending emitter lookup the same walk answers it over [1e-4, ...); a ray that only
+             * carries the lookup needs nothing beyond zfar (next_event_estimation.glsl:5) */
+            const JobView &J = job_of<MULTI>(S, st, slot);
+            trav_init<STACK, kTraceBlock>(w, my, J.tlas_root, O, D, nee ? 0.0001f : 0.001f, 0.001f,
+                      (fl & F_TERMINAL) ? fminf(J.zfar, 10000.0f) : 10000.0f, nee ? fminf(J.zfar, 10000.0f) : 0.001f);
+            active = true;
+            nrays++;
+        }
+        if (__ballot(active) == 0ull && done) break;
+        if (__ballot(active) == 0ull) continue;
+        if (active && trav_step<MODE_CLOSEST2, STACK, kTraceBlock, COUNT>(w, S, my, cnt)) {
+            const TraceHit &h = w.hit;
+            const uint32_t r = 4u * slot;
+            st.hit[r] = make_float4(h.t, h.u, h.v, __uint_as_float(h.prim));
+            st.hit[r + 1] = make_float4(__uint_as_float(h.inst), __uint_as_float(nee ? w.hitA.inst : 0u),
+                                        nee ? w.tskip : 0.0f, 0.0f);
+            if (nee) {
+                st.hit[r + 2] = make_float4(w.hitA.t, w.hitA.u, w.hitA.v, __uint_as_float(w.hitA.prim));
+                st.hit[r + 3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f); /* the whole line, no partial sector */
+            }
+            active = false;
+        }
+    }
+    wave_add64(P.stats, S_PATH, nrays);
+    if (COUNT) {
+        wave_add64(P.stats, S_NODES_EXT, cnt.nodes);
+        wave_add64(P.stats, S_TRIS_EXT, cnt.tris);
+    }
+}
+
 /* ---------------------------------------------------------- k_shade -- */
 struct ShadeOut {
     uint32_t secmask;
@@ -1173,15 +1229,14 @@ __device__ __forceinline__ void job_items_done(const DScene &S, uint32_t job) {
     }
 }
 
-/* Arguments of k_shade and the trace kernels, read where they are used: a by-value kernel argument is loaded whole at the kernel's entry and
+/* Arguments of k_shade, read where they are used: a by-value kernel argument is loaded whole at the kernel's entry and
  * held in scalar registers to its end, and these 900 bytes spilled 229 of them (2,600 v_readlane in the code).  The
  * empty asm keeps the loads behind this point; they are scalar loads from the constant kernel-argument segment. */
-struct LoopArgs {
+struct ShadeArgs {
     DScene S;
     RenderParams P;
     PathState st;
     uint32_t cur;
-    uint32_t phases; /* k_trace8 */
 };
 template <class T>
 __device__ __forceinline__ const T &kernargs() {
@@ -1196,7 +1251,7 @@ __device__ __forceinline__ const T &kernargs() {
 template <bool MULTI, class Fx>
 __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool valid, bool over, bool parked, uint32_t slot,
                                             uint32_t ctr, uint32_t rng_s, f3 L) {
-    const LoopArgs &A = kernargs<LoopArgs>();
+    const ShadeArgs &A = kernargs<ShadeArgs>();
     const DScene &S = A.S;
     const RenderParams &P = A.P;
     const PathState &st = A.st;
@@ -1219,8 +1274,7 @@ __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool vali
     }
     /* finished work items take new ones from the wave's item shard */
     uint32_t ishard = sh, newitem = kInvalid;
-    if (P.items_total > P.nslots) /* else k_init gave every item a slot */
-        item_fetch(P.items, P.items_total, P.items_per_shard, P.item_chunk, item_end, ishard, newitem);
+    item_fetch(P.items, P.items_total, P.items_per_shard, P.item_chunk, item_end, ishard, newitem);
     if (over) {
         const uint32_t item = st.item[slot];
         if (item_end) {
@@ -1276,16 +1330,16 @@ __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool vali
  * arguments read in place took the 1080p field at 64 spp from 152 to 136 ms, the 1080p medium at 32 spp from 202 to
  * 180 ms and a 64x64 preview from 3.2 to 3.0 ms. */
 template <bool MULTI, class Fx>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(LoopArgs) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(ShadeArgs) {
     __shared__ SQView view;
-    const LoopArgs &A0 = kernargs<LoopArgs>();
+    const ShadeArgs &A0 = kernargs<ShadeArgs>();
     const uint32_t cur = A0.cur;
     const uint32_t nxt = cur ^ 1u;
     sq_view_load(A0.P.ext[cur], view);
     const uint32_t count = view.pre[kShards];
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
-        const LoopArgs &A = kernargs<LoopArgs>();
+        const ShadeArgs &A = kernargs<ShadeArgs>();
         const DScene &S = A.S;
         const RenderParams &P = A.P;
         const PathState &st = A.st;
@@ -1598,26 +1652,24 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
     }
 }
 
-/* ----------------------------------------------------------- k_trace -- */
-/* Shadow segments that end at the light or the first occluder (lightSampling.glsl:108-144 when no surface changes
- * volume): persistent walk with lane refill; opaque scenes stop at the first hit, scenes with transparent materials
- * apply the any-hit product of 1 - alpha.  G lanes walk each ray (traverse.h trav_step). */
-template <int STACK, bool COUNT, bool ALPHA, bool MULTI, int G>
-__device__ __forceinline__ void trace_shadows(uint2 *my, uint32_t cur) {
-    const LoopArgs &A = kernargs<LoopArgs>();
-    const DScene &S = A.S;
-    const RenderParams &P = A.P;
-    const PathState &st = A.st;
+/* ---------------------------------------------------------- k_shadow -- */
+/* Shadow segments that end at the light or the first occluder
+ * (lightSampling.glsl:108-144 when no surface changes volume): persistent
+ * walk with lane refill; opaque scenes stop at the first hit, scenes with
+ * transparent materials apply the any-hit product of 1 - alpha. */
+template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
+__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st, uint32_t cur) {
+    __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
+    uint2 *my = stack + threadIdx.x;
     uint32_t nrays = 0;
     TraceCount cnt = {0, 0};
     Trav w;
     ShadowAnyHit ah{&S, 1.0f, false, true};
     bool active = false, done = false;
-    const bool first = (__lane_id() & (G - 1u)) == 0u;
     uint32_t shard = wave_global_id() % kShards, r = 0;
     for (;;) {
         uint32_t v = 0;
-        if (sq_refill<G>(P.shd[cur], !active, shard, done, v) && !active) {
+        if (sq_refill(P.shd[cur], !active, shard, done, v) && !active) {
             r = v;
             const uint32_t x = sec_ix(st, r);
             const float4 o4 = st.sec_o[x], d4 = st.sec_d[x];
@@ -1630,7 +1682,7 @@ __device__ __forceinline__ void trace_shadows(uint2 *my, uint32_t cur) {
             ah.shadowed = false;
             ah.eps_rule = lightseg;
             active = true;
-            if (first) nrays++;
+            nrays++;
         }
         const unsigned long long am = __ballot(active);
         if (am == 0ull) {
@@ -1640,9 +1692,9 @@ __device__ __forceinline__ void trace_shadows(uint2 *my, uint32_t cur) {
         bool fin = false;
         if (active) {
             if (ALPHA)
-                fin = trav_step<MODE_ANYHIT, STACK, kTraceBlock, COUNT, ShadowAnyHit, G>(w, S, my, cnt, &ah);
+                fin = trav_step<MODE_ANYHIT, STACK, kTraceBlock, COUNT, ShadowAnyHit>(w, S, my, cnt, &ah);
             else
-                fin = trav_step<MODE_ANY, STACK, kTraceBlock, COUNT, NoAnyHit, G>(w, S, my, cnt);
+                fin = trav_step<MODE_ANY, STACK, kTraceBlock, COUNT>(w, S, my, cnt);
         }
         if (fin) {
             const bool shadowed = ALPHA ? ah.shadowed : (w.hit.prim != kInvalid);
@@ -1658,10 +1710,8 @@ __device__ __forceinline__ void trace_shadows(uint2 *my, uint32_t cur) {
                 }
             }
             const uint32_t x = sec_ix(st, r);
-            if (first) {
-                const float4 c4 = st.sec_c[x];
-                st.sec_c[x] = st4(isBlack(T) ? mk(0, 0, 0) : ld3(c4) * T, 0.f);
-            }
+            const float4 c4 = st.sec_c[x];
+            st.sec_c[x] = st4(isBlack(T) ? mk(0, 0, 0) : ld3(c4) * T, 0.f);
             active = false;
         }
     }
@@ -1669,109 +1719,6 @@ __device__ __forceinline__ void trace_shadows(uint2 *my, uint32_t cur) {
     if (COUNT) {
         wave_add64(P.stats, S_NODES_SHD, cnt.nodes);
         wave_add64(P.stats, S_TRIS_SHD, cnt.tris);
-    }
-}
-
-/* Closest-hit query of each queued slot's ray, with the previous bounce's emitter lookup where one is pending
- * (MODE_CLOSEST2): persistent walk with lane refill. */
-template <int STACK, bool COUNT, bool MULTI, int G>
-__device__ __forceinline__ void trace_paths(uint2 *my, uint32_t cur) {
-    const LoopArgs &A = kernargs<LoopArgs>();
-    const DScene &S = A.S;
-    const RenderParams &P = A.P;
-    const PathState &st = A.st;
-    uint32_t nrays = 0;
-    TraceCount cnt = {0, 0};
-    Trav w;
-    bool active = false, done = false, nee = false;
-    const bool first = (__lane_id() & (G - 1u)) == 0u;
-    uint32_t shard = wave_global_id() % kShards, slot = 0;
-    for (;;) {
-        uint32_t v = 0;
-        if (sq_refill<G>(P.ext[cur], !active, shard, done, v) && !active && !(v & kParked)) {
-            slot = v;
-            const f3 O = ld3(st.orig[slot]), D = ld3(st.dir[slot]);
-            const uint32_t fl = st.flags[slot];
-            nee = (fl & F_NEE) != 0u;
-            /* with a pending emitter lookup the same walk answers it over [1e-4, ...); a ray that only
-             * carries the lookup needs nothing beyond zfar (next_event_estimation.glsl:5) */
-            const JobView &J = job_of<MULTI>(S, st, slot);
-            trav_init<STACK, kTraceBlock>(w, my, J.tlas_root, O, D, nee ? 0.0001f : 0.001f, 0.001f,
-                      (fl & F_TERMINAL) ? fminf(J.zfar, 10000.0f) : 10000.0f, nee ? fminf(J.zfar, 10000.0f) : 0.001f);
-            active = true;
-            if (first) nrays++;
-        }
-        if (__ballot(active) == 0ull) {
-            if (done) break;
-            continue;
-        }
-        if (active && trav_step<MODE_CLOSEST2, STACK, kTraceBlock, COUNT, NoAnyHit, G>(w, S, my, cnt)) {
-            if (first) {
-                const TraceHit &h = w.hit;
-                const uint32_t r = 4u * slot;
-                st.hit[r] = make_float4(h.t, h.u, h.v, __uint_as_float(h.prim));
-                st.hit[r + 1] = make_float4(__uint_as_float(h.inst), __uint_as_float(nee ? w.hitA.inst : 0u),
-                                            nee ? w.tskip : 0.0f, 0.0f);
-                if (nee) {
-                    st.hit[r + 2] = make_float4(w.hitA.t, w.hitA.u, w.hitA.v, __uint_as_float(w.hitA.prim));
-                    st.hit[r + 3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f); /* the whole line, no partial sector */
-                }
-            }
-            active = false;
-        }
-    }
-    wave_add64(P.stats, S_PATH, nrays);
-    if (COUNT) {
-        wave_add64(P.stats, S_NODES_EXT, cnt.nodes);
-        wave_add64(P.stats, S_TRIS_EXT, cnt.tris);
-    }
-}
-
-/* The queues that this iteration's k_shade fills; their last consumers ran before this iteration's k_trace. */
-__device__ __forceinline__ void reset_next_queues(const RenderParams &P, uint32_t cur) {
-    sq_reset(P.ext[cur ^ 1u]);
-    sq_reset(P.shd[cur ^ 1u]);
-    sq_reset(P.sec);
-    if (P.nrc_use) sq_reset(P.nrcq);
-}
-
-/* The single-segment shadow rays of the previous bounce (kTraceShadows) and the path rays of this one (kTracePaths).
- * Bound by instruction issue and load latency (the geometry is cache-resident): at least 5 waves per SIMD (at most 102
- * VGPRs; 4 otherwise) where the LDS stack allows it (STACK <= 16); 6 waves would spill registers to scratch, and so
- * would both walks in one kernel (34 VGPRs). */
-enum : uint32_t { kTraceShadows = 1u, kTracePaths = 2u };
-template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
-__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(LoopArgs) {
-    __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
-    trace_shadows<STACK, COUNT, ALPHA, MULTI, 1>(stack + threadIdx.x, kernargs<LoopArgs>().cur);
-}
-template <int STACK, bool COUNT, bool MULTI>
-__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(LoopArgs) {
-    __shared__ uint2 stack[(STACK + 3) * kTraceBlock];
-    const LoopArgs &A = kernargs<LoopArgs>();
-    reset_next_queues(A.P, A.cur);
-    trace_paths<STACK, COUNT, MULTI, 1>(stack + threadIdx.x, A.cur);
-}
-
-/* Both queues with eight lanes per ray, for launches with fewer rays than the chip has lanes, which wait for their
- * longest ray: even blocks drain the shadow queue first, odd blocks the extension queue (neither depends on the
- * other), and each then helps with the other, so the launch takes the longer of the two instead of their sum.
- * `phases` leaves a queue out where launches are timed one by one. */
-template <int STACK, bool ALPHA, bool MULTI>
-__global__ __launch_bounds__(kTraceBlock) void k_trace8(LoopArgs) {
-    __shared__ uint2 stack[(STACK + 3) * kTraceBlock];
-    uint2 *my = stack + threadIdx.x;
-    const LoopArgs &A = kernargs<LoopArgs>();
-    const uint32_t cur = A.cur, phases = A.phases;
-    reset_next_queues(A.P, cur);
-    bool shadows = (blockIdx.x & 1u) == 0u;
-    for (int k = 0; k < 2; ++k) {
-        if (shadows) {
-            if (phases & kTraceShadows) trace_shadows<STACK, false, ALPHA, MULTI, 8>(my, cur);
-        } else {
-            if (phases & kTracePaths) trace_paths<STACK, false, MULTI, 8>(my, cur);
-        }
-        shadows = !shadows;
     }
 }
 

@@ -92,22 +92,15 @@ __device__ __forceinline__ uint32_t sq_at(const SQueue &q, const SQView &v, uint
 
 /* Wave-wide search for a shard (starting at `from`) whose counter is below
  * its limit; lane l inspects shard (from + l) % kShards.  Returns kShards if
- * none.  The counters are read racily: the atomic that follows decides.
- * `fresh` reads them with device-scope loads, past the L2 of the wave's own
- * die: atomics from the other dies do not update its lines, so a search after
- * an atomic that got nothing has to look past them, or the wave visits every
- * drained shard in turn, an atomic each (up to 64 at the end of every launch:
- * a 64x64 render took 3.6 ms instead of 2.6).  The first search reads the
- * cached lines, which are enough while shards still hold entries and when
- * everything was drained before the kernel began. */
+ * none.  The counters are read racily: the atomic that follows decides. */
 __device__ __forceinline__ uint32_t find_shard(const uint32_t *ctr, const uint32_t *limit, uint32_t limit_const,
-                                               uint32_t from, bool fresh) {
+                                               uint32_t from) {
     const uint32_t lane = __lane_id();
     const uint32_t s = (from + lane) % kShards;
     bool has = false;
     if (lane < kShards) {
         const uint32_t lim = limit ? limit[s * kPad] : limit_const;
-        has = (fresh ? __hip_atomic_load(ctr + s * kPad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ctr[s * kPad]) < lim;
+        has = ctr[s * kPad] < lim;
     }
     const unsigned long long m = __ballot(has);
     if (m == 0ull) return kShards;
@@ -121,22 +114,18 @@ __device__ __forceinline__ uint32_t find_shard(const uint32_t *ctr, const uint32
  * `shard` and `done` are wave-uniform state owned by the caller.
  */
 constexpr uint32_t kRefill = 16; /* refill once this many lanes of the wave are idle */
-/* G lanes share an entry (idle is the same for all of them): a group counts once, and every lane of it is served. */
-template <uint32_t G = 1>
 __device__ __forceinline__ bool sq_refill(const SQueue &q, bool idle, uint32_t &shard, bool &done, uint32_t &value) {
-    constexpr unsigned long long kLeaders = G == 8 ? 0x0101010101010101ull : ~0ull;
-    static_assert(G == 1 || G == 8, "one lane or eight lanes per entry");
-    unsigned long long im = __ballot(idle) & kLeaders;
-    if (done || (uint32_t)__popcll(im) < kRefill / G) return false;
+    unsigned long long im = __ballot(idle);
+    if (done || (uint32_t)__popcll(im) < kRefill) return false;
     bool got = false;
-    const uint32_t lane = __lane_id() & ~(G - 1u);
+    const uint32_t lane = __lane_id();
     while (im != 0ull && !done) {
         /* shard counts were final when this kernel started (their producers ran before it) */
         const uint32_t n = *sq_count(q, shard);
         const uint32_t req = (uint32_t)__popcll(im);
         const int leader = __ffsll((long long)im) - 1;
         uint32_t base = 0;
-        if ((int)__lane_id() == leader) base = atomicAdd(sq_fetch(q, shard), req);
+        if ((int)lane == leader) base = atomicAdd(sq_fetch(q, shard), req);
         base = __shfl(base, leader);
         const uint32_t take = base < n ? min(n - base, req) : 0u;
         const bool mine = ((im >> lane) & 1ull) != 0ull;
@@ -148,7 +137,7 @@ __device__ __forceinline__ bool sq_refill(const SQueue &q, bool idle, uint32_t &
         }
         im &= ~__ballot(serve); /* served lanes leave the idle mask */
         if (base + req >= n) {  /* drained: find another shard */
-            const uint32_t nx = find_shard(q.fetch, q.count, 0u, shard, take == 0u);
+            const uint32_t nx = find_shard(q.fetch, q.count, 0u, shard);
             if (nx == kShards)
                 done = true;
             else
@@ -182,7 +171,7 @@ __device__ __forceinline__ bool item_fetch(uint32_t *ctr, uint32_t total, uint32
         }
         im &= ~__ballot(serve);
         if (im != 0ull) {
-            const uint32_t nx = find_shard(ctr, nullptr, per, shard, take == 0u);
+            const uint32_t nx = find_shard(ctr, nullptr, per, shard);
             if (nx == kShards) break;
             shard = nx;
         }

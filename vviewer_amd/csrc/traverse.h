@@ -167,50 +167,6 @@ __device__ __forceinline__ uint32_t intersect_node(const WideNode *__restrict__ 
     return hitmask;
 }
 
-/* OR over the eight lanes of a group (lanes 8 k .. 8 k + 7, all active): two quad permutations and a half-row mirror. */
-__device__ __forceinline__ uint32_t or8(uint32_t v) {
-    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, false);  /* quad_perm [1,0,3,2] */
-    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, false);  /* quad_perm [2,3,0,1] */
-    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, false); /* row_half_mirror */
-    return v;
-}
-
-/* intersect_node by a group of eight lanes that hold the same ray: each lane tests one child, with the same
- * arithmetic, and the group combines the masks.  The near and far planes are addressed by the direction's sign
- * (word w2 + 2 k + half of the plane arrays lo x y z, hi x y z). */
-__device__ __forceinline__ uint32_t intersect_node8(const WideNode *__restrict__ nodes, uint32_t idx, f3 O, f3 idir,
-                                                    uint32_t oct_inv, float tmin, float tmax, uint32_t &child_base,
-                                                    uint32_t &leaf_base, uint32_t &imask) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(nodes + idx);
-    const uint32_t child = __lane_id() & 7u, half = child >> 2, sh = 8u * (child & 3u);
-    const uint32_t *q = reinterpret_cast<const uint32_t *>(nodes + idx) + 8 + half;
-    const bool nx = idir.x < 0.0f, ny = idir.y < 0.0f, nz = idir.z < 0.0f;
-    const uint4 w0 = p[0], w1 = p[1];
-    const uint32_t nearx = q[nx ? 6 : 0], farx = q[nx ? 0 : 6];
-    const uint32_t neary = q[ny ? 8 : 2], fary = q[ny ? 2 : 8];
-    const uint32_t nearz = q[nz ? 10 : 4], farz = q[nz ? 4 : 10];
-    const uint32_t ei = w0.w;
-    imask = ei >> 24;
-    child_base = w1.x;
-    leaf_base = w1.y;
-    const float ax = __uint_as_float((ei & 0xffu) << 23) * idir.x, ay = __uint_as_float(((ei >> 8) & 0xffu) << 23) * idir.y,
-                az = __uint_as_float(((ei >> 16) & 0xffu) << 23) * idir.z;
-    const float bx = (__uint_as_float(w0.x) - O.x) * idir.x;
-    const float by = (__uint_as_float(w0.y) - O.y) * idir.y;
-    const float bz = (__uint_as_float(w0.z) - O.z) * idir.z;
-    uint32_t meta = ((half ? w1.w : w1.z) >> sh) & 0xffu;
-    if ((meta & 0x18u) == 0x18u) meta ^= oct_inv; /* an internal child */
-    const float tnx = fmaf((float)((nearx >> sh) & 0xffu), ax, bx);
-    const float tny = fmaf((float)((neary >> sh) & 0xffu), ay, by);
-    const float tnz = fmaf((float)((nearz >> sh) & 0xffu), az, bz);
-    const float tfx = fmaf((float)((farx >> sh) & 0xffu), ax, bx);
-    const float tfy = fmaf((float)((fary >> sh) & 0xffu), ay, by);
-    const float tfz = fmaf((float)((farz >> sh) & 0xffu), az, bz);
-    const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
-    const float tf = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
-    return or8(tn <= tf * 1.000001f ? (meta >> 5) << (meta & 0x1fu) : 0u);
-}
-
 /* Moller-Trumbore with the explicit fma order of the CPU restatement.  A
  * division-free pre-test rejects most misses first; it only rejects when the
  * exact test below would also reject (its margins are far wider than the
@@ -460,40 +416,7 @@ __device__ __forceinline__ void trav_init(Trav &w, uint2 *st, uint32_t root, f3 
  * call that ran a lane's node loop or leaf loop to its end would hold every other lane of the wave until the
  * slowest lane found its next leaf.  The order in which one ray
  * visits nodes and triangles is that of the recursive walk, whatever the interleaving of the wave's lanes. */
-/* A triangle hit at (t, u, v) of the walk's current instance; returns true when it ends the walk. */
-template <int MODE, class AnyHit>
-__device__ __forceinline__ bool trav_candidate(Trav &w, float t, float u, float v, uint32_t prim, AnyHit *anyhit) {
-    if (MODE == MODE_ANY) {
-        if (t >= w.tmin && t <= w.tmax) {
-            w.hit = {t, u, v, w.cur_inst, prim};
-            return true;
-        }
-    } else if (MODE == MODE_ANYHIT) {
-        if (t >= w.tmin && t <= w.tmax) {
-            const TraceHit cand = {t, u, v, w.cur_inst, prim};
-            if ((*anyhit)(cand)) {
-                w.hit = cand;
-                return true;
-            }
-        }
-    } else {
-        if (t >= w.tmin) {
-            if (w.cur_pass)
-                w.tskip = fminf(w.tskip, t);
-            else if (t < w.hitA.t || (t == w.hitA.t && key_less(w.cur_inst, prim, w.hitA.inst, w.hitA.prim)))
-                w.hitA = {t, u, v, w.cur_inst, prim};
-        }
-        if (t >= w.tmin2 && (t < w.hit.t || (t == w.hit.t && key_less(w.cur_inst, prim, w.hit.inst, w.hit.prim))))
-            w.hit = {t, u, v, w.cur_inst, prim};
-    }
-    return false;
-}
-
-/* G = 8: the eight lanes 8 k .. 8 k + 7 walk one ray together, all holding its whole state.  Each tests one child of a
- * node and one triangle of a leaf group; the group's hits are then applied one by one in triangle order by every lane.
- * A step's chain of instructions is a third as long and 8 rays, not 64, diverge in a wave, which is what a launch with
- * fewer rays than the chip has lanes waits for; with more rays the seven lanes that repeat the rest are lost. */
-template <int MODE, int STACK, int BLOCK, bool COUNT, class AnyHit = NoAnyHit, int G = 1>
+template <int MODE, int STACK, int BLOCK, bool COUNT, class AnyHit = NoAnyHit>
 __device__ __forceinline__ bool trav_step(Trav &w, const DScene &S, uint2 *st, TraceCount &cnt,
                                           AnyHit *anyhit = nullptr) {
     if (w.tg.y != 0u && w.in_blas) {
@@ -501,32 +424,7 @@ __device__ __forceinline__ bool trav_step(Trav &w, const DScene &S, uint2 *st, T
          * SAH-collapsed BVH (3 triangle tests per ray): 1 per call 749, 2 730, 3 705 Msamples/s; a second test
          * in the same call mostly runs with the lanes that have no second triangle idle ---- */
         constexpr int kTrisPerStep = 1;
-        if (G == 8) {
-            /* lane j of the group takes the group's j-th pending triangle */
-            const uint32_t sub = __lane_id() & 7u;
-            uint32_t rem = w.tg.y, mine = 0u;
-#pragma unroll
-            for (uint32_t j = 0; j < 8u; ++j) {
-                if (j == sub) mine = rem;
-                rem &= rem - 1u; /* 0 stays 0 */
-            }
-            w.tg.y = rem;
-            const float tcull = (MODE == MODE_CLOSEST2) ? fmaxf(w.hit.t, w.hitA.t) : w.tmax;
-            float t = 0.0f, u = 0.0f, v = 0.0f;
-            uint32_t prim = 0u;
-            bool ok = false;
-            if (mine != 0u) ok = intersect_tri(w.ro, w.rd, S.tris, w.tg.x + __builtin_ctz(mine), tcull, t, u, v, prim);
-            const uint32_t first = __lane_id() & ~7u;
-            uint32_t hits = (uint32_t)(__ballot(ok) >> first) & 0xffu;
-            while (hits != 0u) {
-                const int src = (int)first + __builtin_ctz(hits);
-                hits &= hits - 1u;
-                const float ct = __shfl(t, src), cu = __shfl(u, src), cv = __shfl(v, src);
-                const uint32_t cp = __shfl(prim, src);
-                if (trav_candidate<MODE>(w, ct, cu, cv, cp, anyhit)) return true;
-            }
-        }
-        for (int k = 0; G == 1 && k < kTrisPerStep; ++k) {
+        for (int k = 0; k < kTrisPerStep; ++k) {
             if (w.tg.y == 0u) break;
             const uint32_t bit = __builtin_ctz(w.tg.y);
             w.tg.y &= w.tg.y - 1u;
@@ -536,7 +434,30 @@ __device__ __forceinline__ bool trav_step(Trav &w, const DScene &S, uint2 *st, T
             if (COUNT) cnt.tris++;
             const float tcull = (MODE == MODE_CLOSEST2) ? fmaxf(w.hit.t, w.hitA.t) : w.tmax;
             if (intersect_tri(w.ro, w.rd, S.tris, idx, tcull, t, u, v, prim)) {
-                if (trav_candidate<MODE>(w, t, u, v, prim, anyhit)) return true;
+                if (MODE == MODE_ANY) {
+                    if (t >= w.tmin && t <= w.tmax) {
+                        w.hit = {t, u, v, w.cur_inst, prim};
+                        return true;
+                    }
+                } else if (MODE == MODE_ANYHIT) {
+                    if (t >= w.tmin && t <= w.tmax) {
+                        const TraceHit cand = {t, u, v, w.cur_inst, prim};
+                        if ((*anyhit)(cand)) {
+                            w.hit = cand;
+                            return true;
+                        }
+                    }
+                } else {
+                    if (t >= w.tmin) {
+                        if (w.cur_pass)
+                            w.tskip = fminf(w.tskip, t);
+                        else if (t < w.hitA.t || (t == w.hitA.t && key_less(w.cur_inst, prim, w.hitA.inst, w.hitA.prim)))
+                            w.hitA = {t, u, v, w.cur_inst, prim};
+                    }
+                    if (t >= w.tmin2 &&
+                        (t < w.hit.t || (t == w.hit.t && key_less(w.cur_inst, prim, w.hit.inst, w.hit.prim))))
+                        w.hit = {t, u, v, w.cur_inst, prim};
+                }
             }
         }
         /* a lane whose leaf group is used up goes on to its next node in the same call: the wave runs that node
@@ -601,8 +522,7 @@ __device__ __forceinline__ bool trav_step(Trav &w, const DScene &S, uint2 *st, T
     const float tcull = (MODE == MODE_CLOSEST2) ? fmaxf(w.hit.t, w.hitA.t) : w.tmax;
     uint32_t cb, lb, im;
     if (COUNT) cnt.nodes++;
-    const uint32_t hm = G == 8 ? intersect_node8(S.nodes, node, w.ro, w.idir, w.oct_inv, w.tmin, tcull, cb, lb, im)
-                               : intersect_node(S.nodes, node, w.ro, w.idir, w.oct_inv, w.tmin, tcull, cb, lb, im);
+    const uint32_t hm = intersect_node(S.nodes, node, w.ro, w.idir, w.oct_inv, w.tmin, tcull, cb, lb, im);
     w.ng = make_uint2(cb, (hm & 0xff000000u) | im);
     w.tg = make_uint2(lb, hm & 0x00ffffffu);
     return false;

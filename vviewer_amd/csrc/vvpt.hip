@@ -1148,25 +1148,27 @@ bool with_stack(int stack, F &&f) {
     }
 }
 
-/* Launches the queues named by `phases`; `group`: with eight lanes per ray, in one kernel. */
 template <int STACK, bool MULTI>
-void launch_trace(bool count, bool alpha, bool group, uint32_t phases, dim3 g, hipStream_t s, LoopArgs a) {
-    a.phases = phases;
-    const dim3 b(kTraceBlock);
-    if (group) {
-        if (alpha) hipLaunchKernelGGL((k_trace8<STACK, true, MULTI>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((k_trace8<STACK, false, MULTI>), g, b, 0, s, a);
-        return;
-    }
-    if (phases & kTraceShadows) {
-        if (alpha && count) hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, b, 0, s, a);
-        else if (alpha) hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, b, 0, s, a);
-        else if (count) hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, b, 0, s, a);
-    }
-    if (phases & kTracePaths) {
-        if (count) hipLaunchKernelGGL((k_extend<STACK, true, MULTI>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((k_extend<STACK, false, MULTI>), g, b, 0, s, a);
+void launch_extend(bool count, dim3 g, hipStream_t s, const DScene &S, const RenderParams &P, const PathState &st,
+                   uint32_t cur) {
+    if (count)
+        hipLaunchKernelGGL((k_extend<STACK, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+    else
+        hipLaunchKernelGGL((k_extend<STACK, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+}
+template <int STACK, bool MULTI>
+void launch_shadow(bool count, bool alpha, dim3 g, hipStream_t s, const DScene &S, const RenderParams &P,
+                   const PathState &st, uint32_t cur) {
+    if (alpha) {
+        if (count)
+            hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+        else
+            hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+    } else {
+        if (count)
+            hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+        else
+            hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
     }
 }
 template <int STACK, bool MULTI>
@@ -1242,12 +1244,6 @@ struct JobSpec {
     vvpt_render_info info;
     float *rad, *alb, *nrm;
 };
-
-/* Launches with at most this many live slots per compute unit walk each ray with eight lanes (traverse.h trav_step):
- * at 10,240 path rays and as many shadow rays they make 2,560 waves, 2.5 for each SIMD.  A 64x64 Cornell box (16,384 slots, falling)
- * took 2.12 / 2.03 / 2.29 ms with the line at 20 / 40 / 80 and 2.3 without group walks, the 640x360 field of 10,000
- * instances 8.15 / 8.10 / 8.09 against 8.6 (its tail of few long paths). */
-constexpr uint32_t kGroupRaysPerCU = 40;
 
 /* Items per chunk of a batched render's item order (chunks are dealt round-robin over the item shards). */
 constexpr uint32_t kItemChunk = 4096;
@@ -1605,18 +1601,14 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
          * (same-address atomics) and scans all shards before it ends. */
         uint32_t live = P.nslots;
         dim3 trace_grid, g_shade;
-        bool group_rays = false;
         auto size_grids = [&]() {
-            group_rays = !count_nodes && live <= cus * kGroupRaysPerCU;
-            const uint64_t lanes = (uint64_t)live * (group_rays ? 16u : 1u); /* 8 per path ray and per shadow ray */
-            trace_grid = dim3((uint32_t)std::min<uint64_t>((lanes + kTraceBlock - 1) / kTraceBlock,
-                                                           (uint64_t)cus * c->tune.trace_blocks_per_cu));
+            trace_grid = dim3(std::min<uint32_t>((live + kTraceBlock - 1) / kTraceBlock, cus * c->tune.trace_blocks_per_cu));
             g_shade = dim3(std::min<uint32_t>((live + kBlock - 1) / kBlock, cus * c->tune.shade_blocks_per_cu));
         };
         size_grids();
 
-        /* one wavefront iteration: the general walks of the previous bounce, its shadow rays and the path rays, shade
-         * (+ cache queries).  The general walk serves volume boundaries and transparent surfaces only. */
+        /* one wavefront iteration: the walks of the previous bounce's secondary records, extend, shade (+ cache
+         * queries).  The general walk serves volume boundaries and transparent surfaces only. */
         auto iteration = [&](auto mt, uint32_t cur) -> vvpt_status {
             constexpr bool M = decltype(mt)::value;
             if (walks) {
@@ -1624,24 +1616,15 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                 with_stack(STACK, [&](auto k) { launch_secondary<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st); });
                 HIP_TRY(c, kt.end());
             }
-            auto trace = [&](uint32_t phases) {
-                with_stack(STACK, [&](auto k) {
-                    launch_trace<decltype(k)::value, M>(count_nodes, alpha, group_rays, phases, trace_grid, s, LoopArgs{S, P, st, cur, 0u});
-                });
-            };
-            if (timing) { /* one queue per launch, so that each is timed by itself */
-                HIP_TRY(c, kt.begin(VVPT_K_SHADOW));
-                trace(kTraceShadows);
-                HIP_TRY(c, kt.end());
-                HIP_TRY(c, kt.begin(VVPT_K_EXTEND));
-                trace(kTracePaths);
-                HIP_TRY(c, kt.end());
-            } else {
-                trace(kTraceShadows | kTracePaths);
-            }
+            HIP_TRY(c, kt.begin(VVPT_K_SHADOW));
+            with_stack(STACK, [&](auto k) { launch_shadow<decltype(k)::value, M>(count_nodes, alpha, trace_grid, s, S, P, st, cur); });
+            HIP_TRY(c, kt.end());
+            HIP_TRY(c, kt.begin(VVPT_K_EXTEND));
+            with_stack(STACK, [&](auto k) { launch_extend<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st, cur); });
+            HIP_TRY(c, kt.end());
             HIP_TRY(c, kt.begin(VVPT_K_SHADE));
             with_features<M>(fx, [&](auto f) {
-                hipLaunchKernelGGL((k_shade<M, decltype(f)>), g_shade, dim3(kBlock), 0, s, LoopArgs{S, P, st, cur, 0u});
+                hipLaunchKernelGGL((k_shade<M, decltype(f)>), g_shade, dim3(kBlock), 0, s, ShadeArgs{S, P, st, cur});
             });
             HIP_TRY(c, kt.end());
             if (P.nrc_use) {
