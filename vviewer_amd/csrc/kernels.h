@@ -1324,13 +1324,16 @@ __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool vali
  * its slots to the next extension queue.  A sample that is over but waits for records of its last bounce or for a
  * cache query is parked: its queue entry carries kParked and the next pass ends it.
  *
- * Bound by its dependent gathers (path state, hit, instance, triangle, light) at 3 waves per SIMD: 145 to 168 VGPRs.
+ * Bound by its dependent gathers (path state, hit, instance, triangle, light).  Unconstrained it takes 145 to 168 VGPRs,
+ * 3 waves per SIMD; held to 128 it spills a few and hides more of them with 4 (1080p field 136 -> 129 ms).  With media 3
+ * waves stay better (1080p medium 176.5 against 179.2 ms), and the extended estimator's variants, which hold the sampler's
+ * and the cache's state too and spill most, keep 3 as well.
  * One pass instead of two (a kernel of its own to end samples read the queue, flags and radiance again and wrote them
  * again), code for the scene's features only (textures that are the default texel cost two dependent loads each) and
- * arguments read in place took the 1080p field at 64 spp from 152 to 136 ms, the 1080p medium at 32 spp from 202 to
- * 180 ms and a 64x64 preview from 3.2 to 3.0 ms. */
+ * arguments read in place took the 1080p field at 64 spp from 150 to 136 ms (129 with 4 waves), the 1080p medium at 32
+ * spp from 202 to 180 ms and a 64x64 preview from 3.2 to 3.0 ms. */
 template <bool MULTI, class Fx>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(ShadeArgs) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(Fx::vol || Fx::ext ? 3 : 4, 8))) void k_shade(ShadeArgs) {
     __shared__ SQView view;
     const ShadeArgs &A0 = kernargs<ShadeArgs>();
     const uint32_t cur = A0.cur;
