@@ -38,8 +38,9 @@ constexpr int kTraceBlock = 128;
 /* k_extend and k_shadow: at least 5 waves per SIMD (at most 102 VGPRs; 4 otherwise) where the LDS stack allows it
  * (STACK <= 16).  Their walks wait on dependent node loads, so resident waves hide latency (k_shadow 116 -> 107 ms
  * per 1080p frame at 64 spp; k_extend 67.3 -> 62.4 ms once its world ray and saved TLAS position moved to LDS and it
- * fitted in 92 VGPRs without spilling); 6 waves would spill registers to scratch. */
-#define VVPT_TRACE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(STACK <= 16 ? 5 : 1, 8)))
+ * fitted in 92 VGPRs without spilling); 6 waves would spill registers to scratch, and so would the counting k_extend
+ * at 5. */
+#define VVPT_TRACE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(STACK <= 16 ? (COUNT ? 4 : 5) : 1, 8)))
 constexpr int kBlock = 256;
 
 enum : uint32_t {
@@ -1324,16 +1325,16 @@ __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool vali
  * its slots to the next extension queue.  A sample that is over but waits for records of its last bounce or for a
  * cache query is parked: its queue entry carries kParked and the next pass ends it.
  *
- * Bound by its dependent gathers (path state, hit, instance, triangle, light).  Unconstrained it takes 145 to 168 VGPRs,
- * 3 waves per SIMD; held to 128 it spills a few and hides more of them with 4 (1080p field 136 -> 129 ms).  With media 3
- * waves stay better (1080p medium 176.5 against 179.2 ms), and the extended estimator's variants, which hold the sampler's
- * and the cache's state too and spill most, keep 3 as well.
+ * Bound by its dependent gathers (path state, hit, instance, triangle, light).  It takes 145 to 168 VGPRs, 3 waves per
+ * SIMD, without scratch memory; every variant is held to that.  At 4 waves (128 VGPRs, up to 32 bytes of scratch per
+ * lane) the 1080p field took 129 instead of 132 ms, but both GPU memory faults this kernel's builds have seen came with
+ * variants that spilled, and their cause is not shown.
  * One pass instead of two (a kernel of its own to end samples read the queue, flags and radiance again and wrote them
  * again), code for the scene's features only (textures that are the default texel cost two dependent loads each) and
- * arguments read in place took the 1080p field at 64 spp from 150 to 136 ms (129 with 4 waves), the 1080p medium at 32
+ * arguments read in place took the 1080p field at 64 spp from 150 to 136 ms, the 1080p medium at 32
  * spp from 202 to 180 ms and a 64x64 preview from 3.2 to 3.0 ms. */
 template <bool MULTI, class Fx>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(Fx::vol || Fx::ext ? 3 : 4, 8))) void k_shade(ShadeArgs) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_shade(ShadeArgs) {
     __shared__ SQView view;
     const ShadeArgs &A0 = kernargs<ShadeArgs>();
     const uint32_t cur = A0.cur;

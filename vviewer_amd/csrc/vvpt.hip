@@ -1183,18 +1183,25 @@ void launch_secondary(bool count, dim3 g, hipStream_t s, const DScene &S, const 
 struct RenderFeatures {
     bool ext, nrc, tex, vol;
 };
-/* Calls f(Features<...>()) for the compiled features that cover fx (a batched render has no radiance cache). */
+/* Calls f(Features<...>()) for the compiled features that cover fx.  A batched render has no radiance cache and always
+ * runs the code with media, whatever its jobs: one job of most batches is in one, and the variant of the batched kernel
+ * without media is the one whose first launch ended in a memory fault whose cause is not shown. */
 template <bool MULTI, class F>
 void with_features(const RenderFeatures &fx, F &&f) {
-    auto tv = [&](auto e, auto n) {
-        constexpr bool E = decltype(e)::value, N = decltype(n)::value;
-        if (fx.tex && fx.vol) f(Features<E, N, true, true>());
-        else if (fx.tex) f(Features<E, N, true, false>());
-        else if (fx.vol) f(Features<E, N, false, true>());
-        else f(Features<E, N, false, false>());
-    };
     using T = std::true_type;
     using N = std::false_type;
+    auto tv = [&](auto e, auto n) {
+        constexpr bool E = decltype(e)::value, N_ = decltype(n)::value;
+        if constexpr (MULTI) {
+            if (fx.tex) f(Features<E, N_, true, true>());
+            else f(Features<E, N_, false, true>());
+        } else {
+            if (fx.tex && fx.vol) f(Features<E, N_, true, true>());
+            else if (fx.tex) f(Features<E, N_, true, false>());
+            else if (fx.vol) f(Features<E, N_, false, true>());
+            else f(Features<E, N_, false, false>());
+        }
+    };
     if constexpr (!MULTI) {
         if (fx.nrc) {
             tv(T(), T());
@@ -1548,7 +1555,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     const bool alpha = (S.scene_flags & SCENE_HAS_TRANSPARENT) != 0u;
     /* k_shade queues general walks only for surfaces that change volume or are transparent */
     const bool walks = c->sh.walks;
-    RenderFeatures fx = {ext, nrc, c->sh.textured, (S.scene_flags & SCENE_HAS_VOLUME_CHANGE) != 0u};
+    RenderFeatures fx = {ext, nrc, c->sh.textured, multi || (S.scene_flags & SCENE_HAS_VOLUME_CHANGE) != 0u};
     for (const JobView &j : J) fx.vol = fx.vol || j.cam_volume >= 0;
     P.media = fx.vol ? 1u : 0u;
     /* launch windows: a batched render has one; a single render covers `win` batches per window */
