@@ -248,8 +248,8 @@ const char *vvpt_last_error(const vvpt_ctx *ctx);
  * 985-1018, Open Image Denoise on the host with the radiance, albedo and normal images): this library's own
  * edge-avoiding a-trous wavelet filter on the GPU (Dammertz et al. 2010) over the albedo-demodulated radiance, with
  * edge-stopping weights from the normal and albedo AOVs.  Inputs are width*height RGBA float images as vvpt_render
- * returns them (the normal in its n * 0.5 + 0.5 encoding); out gets the denoised radiance, alpha 1, and may be the
- * radiance buffer itself.  vvpt_denoise takes host buffers, vvpt_denoise_device device buffers on a stream (NULL:
+ * returns them (the normal in its n * 0.5 + 0.5 encoding); out gets the denoised radiance, alpha 1, and may be any
+ * of the three input buffers.  vvpt_denoise takes host buffers, vvpt_denoise_device device buffers on a stream (NULL:
  * the context's). */
 vvpt_status vvpt_denoise(vvpt_ctx *ctx, const float *radiance_rgba, const float *albedo_rgba, const float *normal_rgba,
                          uint32_t width, uint32_t height, float *out_rgba);

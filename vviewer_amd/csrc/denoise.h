@@ -22,7 +22,7 @@ constexpr float kDenoiseSigmaAlbedo = 0.02f; /* surfaces whose albedo differs by
 constexpr float kDenoiseNormalPower = 64.0f;
 
 /* Denoises W x H RGBA float images (device pointers; the normal in the AOV encoding n * 0.5 + 0.5).  tmp holds
- * 2 * W * H float4.  out may alias radiance.  Returns an error message or "". */
+ * 2 * W * H float4.  out may be any of the inputs.  Returns an error message or "". */
 std::string denoise_device(const float *radiance, const float *albedo, const float *normal, uint32_t W, uint32_t H,
                            float *out, float *tmp, hipStream_t stream);
 

@@ -127,8 +127,12 @@ __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *sr
 
 std::string denoise_device(const float *radiance, const float *albedo, const float *normal, uint32_t W, uint32_t H,
                            float *out, float *tmp, hipStream_t s) {
-    /* every level reads what the one before it wrote, the first the radiance; only the last writes out, which may be the
-     * radiance itself */
+    /* Every level reads what the one before it wrote, the first the radiance, and its neighbours' albedo and normals; only
+     * the last writes out.  out may be the radiance itself; where it shares memory with the albedo or the normals, which
+     * other blocks of that level still read, the level goes to tmp and is copied. */
+    const size_t bytes = (size_t)W * H * sizeof(float4);
+    auto shares = [&](const float *in) { return (uintptr_t)in < (uintptr_t)out + bytes && (uintptr_t)out < (uintptr_t)in + bytes; };
+    const bool copy = shares(albedo) || shares(normal);
     float4 *img[2] = {(float4 *)tmp, (float4 *)tmp + (size_t)W * H};
     const float4 *src = (const float4 *)radiance, *alb = (const float4 *)albedo, *nrm = (const float4 *)normal;
     float sc = kDenoiseSigmaColor;
@@ -139,7 +143,7 @@ std::string denoise_device(const float *radiance, const float *albedo, const flo
         const uint32_t tiles_y = ((H + step - 1) / step + kDnTile - 1) / kDnTile;
         const uint32_t nblocks = tiles_x * tiles_y * step * step;
         const dim3 grid((nblocks + 7u) / 8u * 8u), blk(kDnTile * kDnTile);
-        float4 *dst = l + 1 == kDenoiseLevels ? (float4 *)out : img[l & 1];
+        float4 *dst = l + 1 == kDenoiseLevels && !copy ? (float4 *)out : img[l & 1];
         const float inv_sc2 = 1.0f / (sc * sc);
         if (l == 0)
             hipLaunchKernelGGL((k_dn_level<true, false>), grid, blk, 0, s, src, dst, alb, nrm, W, H, (int)step, tiles_x, nblocks, inv_sc2);
@@ -150,7 +154,8 @@ std::string denoise_device(const float *radiance, const float *albedo, const flo
         src = dst;
         sc *= 0.5f;
     }
-    const hipError_t e = hipGetLastError();
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && copy) e = hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToDevice, s);
     return e == hipSuccess ? std::string() : std::string(hipGetErrorString(e));
 }
 
