@@ -17,6 +17,7 @@
  */
 #include "denoise.h"
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -59,9 +60,11 @@ __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *sr
     /* the blocks of one die (block % 8) take consecutive (tile, y class, x class) triples */
     const uint32_t per = (nblocks + 7u) / 8u, lin = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
     if (lin >= nblocks) return;
-    const uint32_t us = (uint32_t)step, rx = lin % us, ry = lin / us % us, tl = lin / (us * us);
+    const uint32_t cx = min((uint32_t)step, W), cy = min((uint32_t)step, H); /* classes that hold a pixel */
+    const uint32_t rx = lin % cx, ry = lin / cx % cy, tl = lin / (cx * cy);
     const int tx = (int)(tl % tiles_x) * kDnTile, ty = (int)(tl / tiles_x) * kDnTile; /* in pixels of the class */
-    for (int k = threadIdx.x; k < kDnHalo * kDnHalo; k += kDnTile * kDnTile) {
+    const int lx = threadIdx.x, ly = threadIdx.y;
+    for (int k = ly * kDnTile + lx; k < kDnHalo * kDnHalo; k += kDnTile * kDnTile) {
         const int qx = (tx + k % kDnHalo - 2) * step + (int)rx, qy = (ty + k / kDnHalo - 2) * step + (int)ry;
         float4 c = make_float4(0.f, 0.f, 0.f, 0.f), t = c, a = make_float4(1e15f, 0.f, 0.f, 0.f);
         float3 n = make_float3(0.f, 0.f, 0.f);
@@ -78,7 +81,6 @@ __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *sr
         tile[2][k] = make_float4(a.z, n.x, n.y, n.z);
     }
     __syncthreads();
-    const int lx = threadIdx.x % kDnTile, ly = threadIdx.x / kDnTile;
     const int x = (tx + lx) * step + (int)rx, y = (ty + ly) * step + (int)ry;
     if (x >= (int)W || y >= (int)H) return;
     const float h[5] = {1.0f / 16.0f, 1.0f / 4.0f, 3.0f / 8.0f, 1.0f / 4.0f, 1.0f / 16.0f};
@@ -141,8 +143,10 @@ std::string denoise_device(const float *radiance, const float *albedo, const flo
         const uint32_t step = 1u << l;
         const uint32_t tiles_x = ((W + step - 1) / step + kDnTile - 1) / kDnTile;
         const uint32_t tiles_y = ((H + step - 1) / step + kDnTile - 1) / kDnTile;
-        const uint32_t nblocks = tiles_x * tiles_y * step * step;
-        const dim3 grid((nblocks + 7u) / 8u * 8u), blk(kDnTile * kDnTile);
+        /* a strip has fewer classes than step * step; blocks of 16 x 16 keep the longest one (2^28 pixels) within the
+         * 2^32 threads a launch may have per axis */
+        const uint32_t nblocks = tiles_x * tiles_y * std::min(step, W) * std::min(step, H);
+        const dim3 grid((nblocks + 7u) / 8u * 8u), blk(kDnTile, kDnTile);
         float4 *dst = l + 1 == kDenoiseLevels && !copy ? (float4 *)out : img[l & 1];
         const float inv_sc2 = 1.0f / (sc * sc);
         if (l == 0)
