@@ -54,8 +54,8 @@ template <bool FIRST, bool LAST>
 __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *src, float4 *dst, const float4 *alb,
                                                                 const float4 *nrm, uint32_t W, uint32_t H, int step,
                                                                 uint32_t tiles_x, uint32_t nblocks, float inv_sc2) {
-    /* a staged pixel: (c, t.x), (t.y, t.z, a.x, a.y), (a.z, n); n = 0 where the pixel saw no surface, and an albedo no
-     * image holds outside the image, whose weight underflows to 0 */
+    /* a staged pixel: (c, t.x), (t.y, t.z, a.x, a.y), (a.z, n); n = 0 where the pixel saw no surface, and NaN outside the
+     * image, which is a zero weight against pixels with and without one */
     __shared__ float4 tile[3][kDnHalo * kDnHalo];
     /* the blocks of one die (block % 8) take consecutive (tile, y class, x class) triples */
     const uint32_t per = (nblocks + 7u) / 8u, lin = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
@@ -66,8 +66,8 @@ __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *sr
     const int lx = threadIdx.x, ly = threadIdx.y;
     for (int k = ly * kDnTile + lx; k < kDnHalo * kDnHalo; k += kDnTile * kDnTile) {
         const int qx = (tx + k % kDnHalo - 2) * step + (int)rx, qy = (ty + k / kDnHalo - 2) * step + (int)ry;
-        float4 c = make_float4(0.f, 0.f, 0.f, 0.f), t = c, a = make_float4(1e15f, 0.f, 0.f, 0.f);
-        float3 n = make_float3(0.f, 0.f, 0.f);
+        float4 c = make_float4(0.f, 0.f, 0.f, 0.f), t = c, a = c;
+        float3 n = make_float3(NAN, NAN, NAN);
         if (qx >= 0 && qx < (int)W && qy >= 0 && qy < (int)H) {
             const size_t q = (size_t)qy * W + qx;
             c = src[q];
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kDnTile * kDnTile) void k_dn_level(const float4 *sr
             const float ax = q1.z - p1.z, ay = q1.w - p1.w, az = q2.x - p2.x;
             const float dc = dx * dx + dy * dy + dz * dz, da = ax * ax + ay * ay + az * az;
             float wn;
-            if (sp) { /* 0 against a pixel without a surface */
+            if (sp) { /* 0 against a pixel without a surface or outside (fmaxf takes the number of a number and NaN) */
                 wn = fmaxf(p2.y * q2.y + p2.z * q2.z + p2.w * q2.w, 0.0f);
                 static_assert(kDenoiseNormalPower == 64.0f, "six squarings");
 #pragma unroll
