@@ -1522,15 +1522,11 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     /* Iteration bound of a launch window (the reference's per-batch fence timeout, :869-876).  A sample lasts at
      * most depth + 2 iterations (one per bounce, a transparent pass-through or a scattering event included, the walk
      * of its last emitter lookup, and one more when it ends with results pending), so a work item needs at most
-     * batch_size (depth + 2) slot-iterations.  While items remain unstarted every slot is busy (k_shade refills a slot in the iteration its item ends),
-     * so a window of total work T slot-iterations on n slots ends within T / n + one item's length; twice that is
-     * the bound.  vvpt_options.max_iterations overrides it. */
+     * batch_size (depth + 2) slot-iterations.  While items remain unstarted every slot is busy (k_shade refills a slot
+     * in the iteration its item ends), so a window of total work T slot-iterations on n slots ends within T / n + one
+     * item's length; twice that is the bound.  vvpt_options.max_iterations replaces it as it is. */
     auto window_bound = [&](uint32_t nb_window) -> uint64_t {
-        if (opt.max_iterations) { /* the option allows a sample depth + 1 iterations: the one it may spend parked comes on top */
-            uint32_t depth = 255u;
-            for (const JobView &j : J) depth = std::min(depth, j.depth);
-            return (uint64_t)std::ceil((double)opt.max_iterations * (depth + 2u) / (depth + 1u));
-        }
+        if (opt.max_iterations) return opt.max_iterations;
         double work = 0.0, tail = 0.0;
         if (multi) {
             for (size_t i = 0; i < njobs; ++i) {
