@@ -54,8 +54,7 @@ constexpr uint32_t kExtendRecords = 1;    /* the slot's ray (each of the two ext
 constexpr uint32_t kSecondaryRecords = 3; /* light-sample segment, emitter lookup of the previous and the last bounce */
 constexpr uint32_t kShadowRecords = 2;    /* light-sample segment, 1 - alpha product in front of a found emitter */
 constexpr uint32_t kQueryRecords = 1;     /* radiance-cache query */
-/* Queue storage in units of kShards * queue_shard_capacity(nslots) entries (the shadow queue is double-buffered: one
- * more kShadowRecords). */
+/* Queue storage in units of kShards * queue_shard_capacity(nslots) entries. */
 constexpr uint32_t kQueueBlocks = 2 * kExtendRecords + kSecondaryRecords + kShadowRecords + kQueryRecords;
 
 

@@ -137,12 +137,11 @@ struct RenderParams {
     uint32_t items_total; /* work items of this launch window (all jobs) */
     uint32_t aovs;
     uint32_t media;    /* a path can be inside a medium (Features::vol): the slots' volumes are kept */
-    uint32_t extended; /* extended mode: scrambled Sobol samples, environment importance sampling */
     uint32_t nslots;
     float total_samples;
     SQueue ext[2]; /* slots with a ray to extend (double-buffered across iterations) */
     SQueue sec;    /* secondary records needing a general walk (3 per slot) */
-    SQueue shd[2]; /* single-segment shadow rays (scenes without volume-changing surfaces), double-buffered like ext */
+    SQueue shd;    /* single-segment shadow rays (scenes without volume-changing surfaces) */
     uint32_t *items; /* kShards padded work-item counters */
     uint32_t items_per_shard;
     uint32_t item_chunk; /* 0: contiguous item shards; else chunks of this many items dealt round-robin */
@@ -698,7 +697,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_extend(DSc
     uint2 *my = stack + threadIdx.x;
     /* the queues that this iteration's k_shade fills; their last consumers ran before this kernel */
     sq_reset(P.ext[cur ^ 1u]);
-    sq_reset(P.shd[cur ^ 1u]);
+    sq_reset(P.shd);
     sq_reset(P.sec);
     if (P.nrc_use) sq_reset(P.nrcq);
     const SQueue &Q = P.ext[cur];
@@ -1383,8 +1382,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3, 8))) 
         const bool tpass = (secmask & F_TPASS) != 0u;
         uint32_t gen = to_shd ? (secmask & ~F_SEC0) : secmask;
         if (tpass) gen &= ~F_SEC1;
-        sq_append(P.shd[nxt], sh, to_shd, slot * 3u);
-        sq_append(P.shd[nxt], sh, tpass, slot * 3u + 1u);
+        sq_append(P.shd, sh, to_shd, slot * 3u);
+        sq_append(P.shd, sh, tpass, slot * 3u + 1u);
         sq_append(P.sec, sh, (gen & F_SEC0) != 0u, slot * 3u + 0u);
         sq_append(P.sec, sh, (gen & F_SEC1) != 0u, slot * 3u + 1u);
         sq_append(P.sec, sh, (gen & F_SEC2) != 0u, slot * 3u + 2u);
@@ -1662,7 +1661,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
  * walk with lane refill; opaque scenes stop at the first hit, scenes with
  * transparent materials apply the any-hit product of 1 - alpha. */
 template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
-__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st, uint32_t cur) {
+__global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st) {
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
     uint2 *my = stack + threadIdx.x;
     uint32_t nrays = 0;
@@ -1673,7 +1672,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DSc
     uint32_t shard = wave_global_id() % kShards, r = 0;
     for (;;) {
         uint32_t v = 0;
-        if (sq_refill(P.shd[cur], !active, shard, done, v) && !active) {
+        if (sq_refill(P.shd, !active, shard, done, v) && !active) {
             r = v;
             const uint32_t x = sec_ix(st, r);
             const float4 o4 = st.sec_o[x], d4 = st.sec_d[x];

@@ -302,7 +302,7 @@ bool material_is_emissive(const vvpt_material &m) {
 }
 
 /* Counter block: count and fetch counters of the queues, and the work-item counters. */
-enum : uint32_t { CB_EXT0 = 0, CB_EXT1 = 2, CB_SEC = 4, CB_SHD0 = 6, CB_SHD1 = 8, CB_ITEMS = 10, CB_NRCQ = 11, CB_N = 13 };
+enum : uint32_t { CB_EXT0 = 0, CB_EXT1 = 2, CB_SEC = 4, CB_SHD = 6, CB_ITEMS = 8, CB_NRCQ = 9, CB_N = 11 };
 constexpr size_t kCounterBytes = (size_t)CB_N * kShards * kPad * sizeof(uint32_t);
 
 /* The environment importance grid of the extended mode: cell weights from the cube map on the device
@@ -1158,17 +1158,17 @@ void launch_extend(bool count, dim3 g, hipStream_t s, const DScene &S, const Ren
 }
 template <int STACK, bool MULTI>
 void launch_shadow(bool count, bool alpha, dim3 g, hipStream_t s, const DScene &S, const RenderParams &P,
-                   const PathState &st, uint32_t cur) {
+                   const PathState &st) {
     if (alpha) {
         if (count)
-            hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+            hipLaunchKernelGGL((k_shadow<STACK, true, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
         else
-            hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+            hipLaunchKernelGGL((k_shadow<STACK, false, true, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
     } else {
         if (count)
-            hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+            hipLaunchKernelGGL((k_shadow<STACK, true, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
         else
-            hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st, cur);
+            hipLaunchKernelGGL((k_shadow<STACK, false, false, MULTI>), g, dim3(kTraceBlock), 0, s, S, P, st);
     }
 }
 template <int STACK, bool MULTI>
@@ -1372,7 +1372,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
      * per slot and the shadow queue two (a slot's light-sample segment and the 1 - alpha product in front of the
      * emitter its previous bounce found through a transparent surface can both be queued in one iteration). */
     const uint32_t cap1 = queue_shard_capacity(N);
-    HIP_TRY(c, ensure(c->queues, (size_t)kShards * cap1 * (kQueueBlocks + kShadowRecords) * sizeof(uint32_t)));
+    HIP_TRY(c, ensure(c->queues, (size_t)kShards * cap1 * kQueueBlocks * sizeof(uint32_t)));
     HIP_TRY(c, ensure(c->counters, kCounterBytes));
     HIP_TRY(c, ensure(c->stats, (size_t)kShards * kStatStride * sizeof(unsigned long long)));
     HIP_TRY(c, ensure(c->partials, (size_t)items_max * sizeof(float4) * (aovs ? 3 : 1)));
@@ -1407,7 +1407,6 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     RenderParams P;
     std::memset(&P, 0, sizeof(P));
     P.aovs = aovs ? 1u : 0u;
-    P.extended = ext ? 1u : 0u;
     uint32_t *q = (uint32_t *)c->queues.p;
     uint32_t *cb = (uint32_t *)c->counters.p;
     auto mkq = [&](uint32_t *data, uint32_t cap, uint32_t slot) {
@@ -1421,8 +1420,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
     P.ext[0] = mkq(q, kExtendRecords * cap1, CB_EXT0);
     P.ext[1] = mkq(q + (size_t)kShards * cap1, kExtendRecords * cap1, CB_EXT1);
     P.sec = mkq(q + (size_t)2 * kShards * cap1, kSecondaryRecords * cap1, CB_SEC);
-    P.shd[0] = mkq(q + (size_t)(2 + kSecondaryRecords) * kShards * cap1, kShadowRecords * cap1, CB_SHD0);
-    P.shd[1] = mkq(q + (size_t)kQueueBlocks * kShards * cap1, kShadowRecords * cap1, CB_SHD1);
+    P.shd = mkq(q + (size_t)(2 + kSecondaryRecords) * kShards * cap1, kShadowRecords * cap1, CB_SHD);
     if (nrc) {
         /* radiance cache: training blocks of up to min(depth, 16) vertices, 65536 training samples per frame,
          * one query slot per path slot */
@@ -1620,7 +1618,7 @@ vvpt_status render_core(vvpt_ctx *c, const std::vector<JobSpec> &jobs, bool mult
                 HIP_TRY(c, kt.end());
             }
             HIP_TRY(c, kt.begin(VVPT_K_SHADOW));
-            with_stack(STACK, [&](auto k) { launch_shadow<decltype(k)::value, M>(count_nodes, alpha, trace_grid, s, S, P, st, cur); });
+            with_stack(STACK, [&](auto k) { launch_shadow<decltype(k)::value, M>(count_nodes, alpha, trace_grid, s, S, P, st); });
             HIP_TRY(c, kt.end());
             HIP_TRY(c, kt.begin(VVPT_K_EXTEND));
             with_stack(STACK, [&](auto k) { launch_extend<decltype(k)::value, M>(count_nodes, trace_grid, s, S, P, st, cur); });
