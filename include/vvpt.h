@@ -199,9 +199,9 @@ typedef struct {
 /* Per-render counters, filled by vvpt_render*(). */
 typedef enum {
     VVPT_K_EXTEND = 0,    /* closest-hit extension of path rays */
-    VVPT_K_SHADE = 1,     /* one bounce of the hit / miss shaders */
+    VVPT_K_SHADE = 1,     /* one bounce of the hit / miss shaders; sample ends, work-item refill, queue compaction */
     VVPT_K_SECONDARY = 2, /* emitter lookups and multi-segment shadow walks */
-    VVPT_K_FINISH = 3,    /* sample end, work-item refill, queue compaction */
+    VVPT_K_FINISH = 3,    /* no launches of its own any more (its work is in VVPT_K_SHADE): always 0 */
     VVPT_K_SHADOW = 4,    /* single-segment shadow rays */
     VVPT_K_NRC = 5,       /* radiance-cache queries and training */
     VVPT_K_COUNT = 6

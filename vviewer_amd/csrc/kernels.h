@@ -1326,8 +1326,8 @@ __device__ __forceinline__ void end_samples(uint32_t nxt, uint32_t sh, bool vali
  *
  * Bound by its dependent gathers (path state, hit, instance, triangle, light).  It takes 145 to 168 VGPRs, 3 waves per
  * SIMD, without scratch memory; every variant is held to that.  At 4 waves (128 VGPRs, up to 32 bytes of scratch per
- * lane) the 1080p field took 129 instead of 132 ms, but both GPU memory faults this kernel's builds have seen came with
- * variants that spilled, and their cause is not shown.
+ * lane) the benchmark's 1080p field took 138.6 instead of 140.0 ms a frame, but both GPU memory faults this kernel's
+ * builds have seen came with variants that spilled, and their cause is not shown.
  * One pass instead of two (a kernel of its own to end samples read the queue, flags and radiance again and wrote them
  * again), code for the scene's features only (textures that are the default texel cost two dependent loads each) and
  * arguments read in place took the 1080p field at 64 spp from 150 to 136 ms, the 1080p medium at 32

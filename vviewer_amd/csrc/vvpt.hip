@@ -1184,8 +1184,8 @@ struct RenderFeatures {
     bool ext, nrc, tex, vol;
 };
 /* Calls f(Features<...>()) for the compiled features that cover fx.  A batched render has no radiance cache and always
- * runs the code with media, whatever its jobs: one job of most batches is in one, and the variant of the batched kernel
- * without media is the one whose first launch ended in a memory fault whose cause is not shown. */
+ * runs the code with media, whatever its jobs: most batches hold a job in one, and the batched variant without media is
+ * the one whose first launch through a captured graph ended in a memory fault whose cause is not shown. */
 template <bool MULTI, class F>
 void with_features(const RenderFeatures &fx, F &&f) {
     using T = std::true_type;
