@@ -1660,6 +1660,15 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
  * (lightSampling.glsl:108-144 when no surface changes volume): persistent
  * walk with lane refill; opaque scenes stop at the first hit, scenes with
  * transparent materials apply the any-hit product of 1 - alpha. */
+/* k_shadow's arguments in place: its queue is read where lanes refill.  Held in scalar registers it spilled 38 of them in
+ * the batched kernel with alpha (8 this way): 24 jobs 66.3 -> 65.0 ms. */
+struct TraceArgs {
+    DScene S;
+    RenderParams P;
+    PathState st;
+};
+static_assert(sizeof(DScene) % alignof(RenderParams) == 0 && sizeof(RenderParams) % alignof(PathState) == 0,
+              "laid out as the kernel's three arguments");
 template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
 __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st) {
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
@@ -1672,7 +1681,7 @@ __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DSc
     uint32_t shard = wave_global_id() % kShards, r = 0;
     for (;;) {
         uint32_t v = 0;
-        if (sq_refill(P.shd, !active, shard, done, v) && !active) {
+        if (sq_refill(kernargs<TraceArgs>().P.shd, !active, shard, done, v) && !active) {
             r = v;
             const uint32_t x = sec_ix(st, r);
             const float4 o4 = st.sec_o[x], d4 = st.sec_d[x];
