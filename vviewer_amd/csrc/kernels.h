@@ -1656,10 +1656,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_secondary(DScene S, RenderParam
 }
 
 /* ---------------------------------------------------------- k_shadow -- */
-/* Shadow segments that end at the light or the first occluder
- * (lightSampling.glsl:108-144 when no surface changes volume): persistent
- * walk with lane refill; opaque scenes stop at the first hit, scenes with
- * transparent materials apply the any-hit product of 1 - alpha. */
 /* k_shadow's arguments in place: its queue is read where lanes refill.  Held in scalar registers it spilled 38 of them in
  * the batched kernel with alpha (8 this way): 24 jobs 66.3 -> 65.0 ms. */
 struct TraceArgs {
@@ -1669,6 +1665,10 @@ struct TraceArgs {
 };
 static_assert(sizeof(DScene) % alignof(RenderParams) == 0 && sizeof(RenderParams) % alignof(PathState) == 0,
               "laid out as the kernel's three arguments");
+/* Shadow segments that end at the light or the first occluder
+ * (lightSampling.glsl:108-144 when no surface changes volume): persistent
+ * walk with lane refill; opaque scenes stop at the first hit, scenes with
+ * transparent materials apply the any-hit product of 1 - alpha. */
 template <int STACK, bool COUNT, bool ALPHA, bool MULTI>
 __global__ __launch_bounds__(kTraceBlock) VVPT_TRACE_OCCUPANCY void k_shadow(DScene S, RenderParams P, PathState st) {
     __shared__ uint2 stack[(STACK + 3) * kTraceBlock]; /* the walk stack + the world ray */
